@@ -301,7 +301,7 @@ struct qb_problem {
     DevProblem dev{};
     int n = 0, n_rays = 0, n_classes = 0;
     int64_t nnz = 0, n_nbr = 0;
-    int max_class = 0, min_class = 0, max_entries = 0, max_bits_per_ray = 0;
+    int max_class = 0, min_class = 0, max_entries = 0, max_bits_per_ray = 0, max_nbr = 0;
     int64_t device_bytes = 0;
     std::vector<int32_t> pos_bit, cls_ptr;
     DevBuf b_cls, b_pos, b_col, b_ent, b_nbp, b_nb, b_nbbit, b_lin, b_d, b_w, b_rtp, b_rt, b_seq, b_dbit, b_dkey,
@@ -314,6 +314,12 @@ struct qb_problem {
         DevBatches dev{};
     };
     std::map<int, std::unique_ptr<Batches>> batches;   // by group width and team size
+    struct Solo {
+        DevBuf lists, blk, cls_draw, wide;
+        DevSolo dev{};
+    };
+    std::unique_ptr<Solo> solo;   // the one-workgroup-per-branch plan, made on first use
+    double solo_us = -1.0;        // its estimated time per sweep, < 0 until asked for
     // workspace
     DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_rref,
         w_rng, w_energy;
@@ -586,6 +592,7 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
     QB_HIP(hipStreamSynchronize(st));
     P->col_ptr = col_ptr;
     P->nb_ptr = nb_ptr;
+    for (int p = 0; p < n; ++p) P->max_nbr = std::max(P->max_nbr, nb_ptr[size_t(p) + 1] - nb_ptr[size_t(p)]);
     P->seq_update = seq_update;
     P->light_begin = light_begin;
     P->device_bytes = int64_t(P->b_dbit.bytes + P->b_dkey.bytes + P->b_lbeg.bytes + P->b_lnb.bytes +
@@ -853,6 +860,218 @@ static int batches_for(qb_problem* P, int bw, int team_size, const DevBatches** 
     return QB_OK;
 }
 
+// Chains of the longest bit when it has more than kSoloChains of them (a wide bit), else 0.
+static int solo_wide_chains(const qb_problem* P) {
+    const int most = (P->max_entries + kSeg - 1) / kSeg;
+    return most > kSoloChains ? most : 0;
+}
+
+// Microseconds of one sweep in the solo kernel, from its measured parts: 0.75 per class (a
+// class with a tile or two per wave), 0.13 per further tile of 32 chains (0.2 where the
+// tiles are too many for the caches), 0.2 per tile of 64 ray-free bits, 2 per wide bit.
+// Within 15% of the kernel on muon problems of 2k to 306k bits (22 classes x 0.95 us to
+// 97 x 11.7 us) and gravimetry problems of 3k to 200k cells (135 x 0.85 us to 2,586 x 9.1 us).
+static double solo_sweep_us(const qb_problem* P) {
+    double light = 0.0, wide = 0.0, small_tiles = 0.0, tiles = 0.0;
+    for (int c = 0; c < P->n_classes; ++c) {
+        int total = 0, long_bits = 0, rest = 0, free_bits = 0;
+        for (int q = P->cls_ptr[size_t(c)]; q < P->cls_ptr[size_t(c) + 1]; ++q) {
+            const int e = P->col_ptr[size_t(q) + 1] - P->col_ptr[size_t(q)], k = (e + kSeg - 1) / kSeg;
+            if (e == 0) ++free_bits;
+            else if (k > kSoloChains) wide += 1.0;
+            else if (k > 16) ++long_bits;
+            else rest += k;
+            if (k <= kSoloChains) total += k;
+        }
+        light += double((free_bits + 63) / 64);
+        if (total > 16 * kSoloStepWaves) tiles += double(long_bits + (rest + 31) / 32);
+        else small_tiles += double(long_bits);
+    }
+    const bool streamed = tiles * double(solo_tile_bytes(2)) > 128e6;
+    return 0.75 * P->n_classes + (streamed ? 0.2 : 0.13) * (tiles + small_tiles) + 0.2 * light + 2.0 * wide;
+}
+
+// Whether the anneal runs one workgroup per branch (ray_solo_kernel) on `cus` compute units.
+// The branch's residuals and spins must fit one CU's LDS; the caller's explicit launch
+// shapes (workgroups, group_width) name the team kernel; so do the neighbour lists and class
+// counts past its limits, which it refuses. Where both can run, the shorter estimate
+// decides: the solo kernel's sweep above, once per `cus` branches, against the team
+// kernel's classes, each 4.5 us for up to 16 branches and more beyond with the branches and
+// the class's chains (measured: 4.3 to 5.5 us at 16 branches; at 256, 10.6 us with 41
+// chains a class to 25 us with 1,077). At 16 branches the two meet near 400 chains a class.
+static bool solo_fits(qb_problem* P, const qb_anneal_opts& o, int R, int cus) {
+    if (o.workgroups != 0 || o.group_width != 0 || P->n <= 0 || P->n_classes <= 0) return false;
+    if (sweep_table_bytes(P->n_classes) > size_t(kSweepTableLimit)) return false;
+    if (P->max_nbr > kMaxPackedNeighbours || solo_wide_chains(P) > kSoloBlock * kChainRun) return false;
+    if (solo_dynamic_lds(P->n, P->n_rays, solo_wide_chains(P), o.precision, true) > solo_lds_limit()) return false;
+    if (P->solo_us < 0.0) P->solo_us = solo_sweep_us(P);
+    const double solo = P->solo_us * double((R + cus - 1) / cus);
+    const double chains = double(P->nnz) / kSeg / P->n_classes;
+    const double team = P->n_classes * (4.5 + std::max(0, R - 16) * (0.022 + 6e-5 * chains));
+    return solo < team;
+}
+
+// Packs every class's bits into one-wave tiles and deals them to the waves. A class's
+// bits with entries, longest first, go to the least filled tile that has room: as few tiles
+// of four lanes a chain as hold them while there is a wave for each, else (and for bits of
+// more than 16 chains) tiles of two lanes a chain, which issue fewer instructions in all.
+// Ray-free bits fill tiles of their own. A tile goes to the wave with the least work of the
+// class so far.
+static int solo_for(qb_problem* P, const DevSolo** out) {
+    if (P->solo) {
+        *out = &P->solo->dev;
+        return QB_OK;
+    }
+    constexpr int kWaves = kSoloStepWaves;
+    const int K = P->n_classes;
+    auto entries = [&](int q) { return P->col_ptr[size_t(q) + 1] - P->col_ptr[size_t(q)]; };
+    auto chains = [&](int q) { return std::max(1, (entries(q) + kSeg - 1) / kSeg); };
+    auto kind_of = [](int lpc) { return lpc == 4 ? 0 : lpc == 2 ? 1 : 2; };
+    struct Bin {
+        std::vector<int> bits;
+        int used = 0, lpc = 1;
+    };
+    std::vector<SoloWide> wide;
+    std::vector<int2> cls_draw;
+    std::vector<SoloTile> tiles[kSoloWaves][3];   // next_cls holds the tile's own class until the lists are whole
+    std::vector<SlotDesc> desc;
+    std::vector<Bin> bins;
+    std::vector<int> normal, light;
+    for (int c = 0; c < K; ++c) {
+        const int p0 = P->cls_ptr[size_t(c)], p1 = P->cls_ptr[size_t(c) + 1];
+        normal.clear();
+        light.clear();
+        bins.clear();
+        int total = 0;
+        for (int q = p0; q < p1; ++q) {
+            if (chains(q) > kSoloChains) {
+                SoloWide w{};
+                w.cls = c;
+                w.pos = q;
+                w.k0 = P->col_ptr[size_t(q)];
+                w.k1 = P->col_ptr[size_t(q) + 1];
+                w.nn = P->nb_ptr[size_t(q) + 1] - P->nb_ptr[size_t(q)];
+                w.seq = P->seq_update[size_t(q)] ? 1 : 0;
+                wide.push_back(w);   // the device fills in the rest
+            } else if (entries(q) == 0) {
+                light.push_back(q);
+            } else {
+                normal.push_back(q);
+                total += chains(q);
+            }
+        }
+        cls_draw.push_back(int2{p0, std::min(P->light_begin[size_t(c)] - p0, kSoloDraws)});
+        std::stable_sort(normal.begin(), normal.end(), [&](int a, int b) { return chains(a) > chains(b); });
+        auto pack = [&](size_t begin, size_t end, int lpc) {
+            const int room = 64 / lpc;
+            int sum = 0;
+            for (size_t i = begin; i < end; ++i) sum += chains(normal[i]);
+            const size_t b0 = bins.size();
+            if (begin < end) bins.resize(b0 + size_t((sum + room - 1) / room));
+            for (size_t t = b0; t < bins.size(); ++t) bins[t].lpc = lpc;
+            size_t open = b0;   // with many tiles, fill them in turn
+            for (size_t i = begin; i < end; ++i) {
+                const int k = chains(normal[i]);
+                size_t best = open;
+                if (bins.size() - b0 <= size_t(kWaves)) {
+                    for (size_t t = b0 + 1; t < bins.size(); ++t)
+                        if (bins[t].used < bins[best].used) best = t;
+                }
+                if (bins[best].used + k > room) {
+                    if (bins.size() - b0 > size_t(kWaves) && open + 1 < bins.size()) {
+                        best = ++open;
+                    } else {
+                        bins.emplace_back();
+                        best = bins.size() - 1;
+                        bins[best].lpc = lpc;
+                        if (bins.size() - b0 > size_t(kWaves)) open = best;
+                    }
+                }
+                bins[best].bits.push_back(normal[i]);
+                bins[best].used += k;
+            }
+        };
+        size_t n_long = 0;   // bits too long for four lanes a chain lead the order
+        while (n_long < normal.size() && chains(normal[n_long]) > 16) ++n_long;
+        if (total <= 16 * kWaves) {
+            pack(0, n_long, 2);
+            pack(n_long, normal.size(), 4);
+        } else {
+            pack(0, normal.size(), 2);
+        }
+        for (size_t i = 0; i < light.size(); i += 64) {
+            bins.emplace_back();
+            bins.back().bits.assign(light.begin() + int64_t(i),
+                                    light.begin() + int64_t(std::min(light.size(), i + 64)));
+            bins.back().used = int(bins.back().bits.size());
+        }
+        int64_t load[kSoloWaves] = {};
+        for (int w = kWaves; w < kSoloWaves; ++w)   // a draw wave's chunks of the next class's draws
+            load[w] = 2 * ((P->light_begin[size_t(c + 1 < K ? c + 1 : 0)] - P->cls_ptr[size_t(c + 1 < K ? c + 1 : 0)] +
+                            64 * kSoloDrawWaves - 1) / (64 * kSoloDrawWaves));
+        for (const Bin& b : bins) {
+            if (b.bits.empty()) continue;
+            SoloTile t{};
+            t.next_cls = c;
+            t.lpc = int16_t(b.lpc);
+            t.chains = int16_t(b.used);
+            t.chain0 = int32_t(desc.size());
+            for (int q : b.bits) {
+                const int k0 = P->col_ptr[size_t(q)], nch = chains(q);
+                const int nn = P->nb_ptr[size_t(q) + 1] - P->nb_ptr[size_t(q)];
+                if (nch > 1) t.flags |= kSoloMulti;
+                if (nch > 4) t.flags |= kSoloHalf;
+                if (nch > kChainRun) t.flags |= kSoloRuns;
+                if (P->seq_update[size_t(q)]) t.flags |= kSoloSeq;
+                if (b.lpc > 1 && q - p0 >= kSoloDraws) t.flags |= kSoloOwn;
+                for (int j = 0; j < nch; ++j) {
+                    const int len = std::max(0, std::min(kSeg, entries(q) - j * kSeg));
+                    desc.push_back(SlotDesc{q, k0 + j * kSeg, std::min(q - p0, kSoloDraws - 1),
+                                            uint32_t(len) | (uint32_t(j) << 5) | (uint32_t(nch) << 13) |
+                                                (uint32_t(nn) << 21) |
+                                                (uint32_t(P->seq_update[size_t(q)] ? 1u : 0u) << 31)});
+                }
+            }
+            const int w = int(std::min_element(load, load + (b.lpc == 1 ? kSoloWaves : kWaves)) - load);
+            tiles[w][kind_of(b.lpc)].push_back(t);
+            load[w] += 2 + (b.lpc == 2 ? 1 : 0) + ((t.flags & kSoloRuns) ? 1 : 0);
+        }
+    }
+    // the lists one after another; each tile carries the class of its list's next one
+    std::vector<SoloTile> all;
+    std::vector<SoloLists> lists(static_cast<size_t>(kSoloWaves));
+    int64_t bytes = 0;
+    for (int w = 0; w < kSoloWaves; ++w)
+        for (int lpc : {4, 2, 1}) {
+            std::vector<SoloTile>& l = tiles[w][kind_of(lpc)];
+            lists[size_t(w)].at[kind_of(lpc)] = bytes;
+            lists[size_t(w)].n[kind_of(lpc)] = int32_t(l.size());
+            lists[size_t(w)].cls[kind_of(lpc)] = l.empty() ? -1 : l[0].next_cls;
+            const int first = l.empty() ? -1 : l[0].next_cls;
+            for (size_t i = 0; i < l.size(); ++i) {
+                l[i].next_cls = i + 1 < l.size() ? l[i + 1].next_cls : first;
+                l[i].at = bytes;
+                bytes += solo_tile_bytes(lpc);
+                all.push_back(l[i]);
+            }
+        }
+    auto S = std::make_unique<qb_problem::Solo>();
+    DevBuf d_tiles, d_desc;
+    int rc;
+    if ((rc = S->lists.upload(lists, P->stream)) || (rc = S->wide.upload(wide, P->stream)) ||
+        (rc = S->cls_draw.upload(cls_draw, P->stream)) || (rc = d_tiles.upload(all, P->stream)) ||
+        (rc = d_desc.upload(desc, P->stream)) || (rc = S->blk.reserve(size_t(std::max<int64_t>(bytes, 1)))))
+        return rc;
+    QB_HIP(launch_solo_blocks(P->dev, d_tiles.as<SoloTile>(), d_desc.as<SlotDesc>(), int(all.size()), S->blk.p,
+                              S->wide.as<SoloWide>(), int(wide.size()), P->stream));
+    QB_HIP(hipStreamSynchronize(P->stream));
+    S->dev = DevSolo{S->blk.p, S->lists.as<SoloLists>(), S->cls_draw.as<int2>(), S->wide.as<SoloWide>(), int(wide.size()),
+                     solo_wide_chains(P)};
+    *out = &S->dev;
+    P->solo = std::move(S);
+    return QB_OK;
+}
+
 extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, uint64_t seed_offset,
                                   const qb_anneal_opts* opts, uint8_t* branches, float* p_void, uint8_t* tri,
                                   float* certainty, double* energy, qb_report* rep) {
@@ -869,14 +1088,19 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
         return fail(QB_E_ARG, "group_width must be 0, 2, 4, 8 or 16 (got %d)", o.group_width);
     const int total = s->anneal_sweeps + s->hold_sweeps;
     const int n = P->n, nr = P->n_rays;
-    const int bw = group_width_for(P, R, o.group_width, o.precision);
+    const int team_bw = group_width_for(P, R, o.group_width, o.precision);
+    const int team_size = team_size_for(o.workgroups, o.precision, team_bw, 0);
+    if (team_size <= 0) return -team_size;
+    const bool solo = solo_fits(P, o, R, 8 * team_size);
+    const int bw = solo ? 1 : team_bw;
     const int n_groups = (R + bw - 1) / bw;
     const size_t tsz = o.precision == QB_FP32 ? sizeof(float) : sizeof(double);
-    const int team_size = team_size_for(o.workgroups, o.precision, bw, 0);
-    if (team_size <= 0) return -team_size;
     const DevBatches* bt = nullptr;
-    if ((rc = batches_for(P, bw, team_size, &bt))) return rc;
-    {
+    const DevSolo* sp = nullptr;
+    if (solo) {
+        if ((rc = solo_for(P, &sp))) return rc;
+    } else {
+        if ((rc = batches_for(P, bw, team_size, &bt))) return rc;
         // the dynamic LDS must not lower the residency the team size was chosen for
         const int checked =
             team_size_for(o.workgroups, o.precision, bw, sweep_dynamic_lds(P->n_classes, bw, bt->heavy_lds != 0, o.precision));
@@ -900,18 +1124,23 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
     QB_HIP(hipStreamSynchronize(st));
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(P->w_beta.p, beta.data(), sizeof(double) * beta.size(), hipMemcpyHostToDevice, st));
-    QB_HIP(launch_ray_init(P->dev, o.precision, bw, P->w_x.p, P->w_r.p, n_groups, st));
+    if (!solo) QB_HIP(launch_ray_init(P->dev, o.precision, bw, P->w_x.p, P->w_r.p, n_groups, st));
     QB_HIP(hipMemsetAsync(P->w_err.p, 0, sizeof(int), st));
     const int chunk = o.sweeps_per_launch > 0 ? std::min(o.sweeps_per_launch, total) : total;
     int launches = 0;
     QB_HIP(hipEventRecord(P->ev0, st));
     for (int sb = 0; sb < total; sb += chunk) {
+        ++launches;
+        if (solo) {
+            QB_HIP(launch_ray_solo(P->dev, *sp, o.precision, P->w_x.p, P->w_r.p, R, seed_offset,
+                                   P->w_beta.as<double>(), sb, std::min(total, sb + chunk), o.recompute_every, st));
+            continue;
+        }
         QB_HIP(hipMemsetAsync(P->w_bar.p, 0, sizeof(unsigned) * (kBarWords + kTicketWords), st));
         QB_HIP(launch_ray_sweeps(P->dev, *bt, o.precision, bw, P->w_x.p, P->w_r.p, n_groups, R, seed_offset,
                                  P->w_beta.as<double>(), sb, std::min(total, sb + chunk), o.recompute_every,
                                  P->w_bar.as<unsigned>(), P->w_bar.as<unsigned>() + kBarWords, P->w_err.as<int>(),
                                  team_size, st));
-        ++launches;
     }
     QB_HIP(hipEventRecord(P->ev1, st));
     const bool want_outputs = p_void || tri || certainty || branches;

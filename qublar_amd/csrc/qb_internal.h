@@ -182,6 +182,62 @@ struct DevGraph {
     const int32_t* ew;
 };
 
+// ---- small problems: one workgroup per branch (qb_solo.hip) ----
+// A tile is one step wave's unit of work in a class: 64 lanes, lpc of them (4 or 2) per chain
+// of one bit, or one per ray-free bit (lpc 1). Its layout is fixed: the heads' planes, one
+// 16-byte granule per chain, then kSeg / lpc planes of entries, one per lane. A head's first
+// granule is {position, info, class of the list's next tile, the draw's slot}, info a
+// SlotDesc's with the tile's flags in place of the length.
+constexpr int solo_tile_bytes(int lpc) {
+    return lpc == 1 ? 4 * 64 * 16 : 3 * (64 / lpc) * 16 + (kSeg / lpc) * 64 * 16;
+}
+struct SoloTile {            // a tile to be written
+    int64_t at;              // its byte offset
+    int32_t chain0, next_cls;
+    int16_t chains, lpc;
+    int32_t flags;
+};
+struct SoloWide {            // a wide bit
+    int32_t cls, pos, k0, k1, nn, seq, bit;
+    int32_t q[kNb];          // first neighbour positions (the last repeated past the bit's count)
+    int32_t pad;
+    double lin;
+    uint64_t key;
+};
+struct SoloLists {           // one wave's tiles with lpc 4, 2 (step waves) and 1
+    int64_t at[3];           // byte offset of the first
+    int32_t n[3], cls[3];    // tiles, and the first one's class
+};
+constexpr int kSoloMulti = 1;   // some bit of the tile has more than one chain
+constexpr int kSoloHalf = 2;    // some bit has more than four chains
+constexpr int kSoloRuns = 4;    // some bit has more than kChainRun chains
+constexpr int kSoloSeq = 8;     // some bit's column repeats a ray
+constexpr int kSoloOwn = 16;    // some bit's draw is not made ahead
+constexpr int kSoloStepWaves = 6;
+constexpr int kSoloDrawWaves = 2;
+constexpr int kSoloWaves = kSoloStepWaves + kSoloDrawWaves;
+constexpr int kSoloBlock = 64 * kSoloWaves;
+constexpr int kSoloDraws = 384;   // draws made ahead per class
+constexpr int kSoloChains = 32;   // a bit with more chains is wide
+constexpr int kSoloPart = 64;     // a wave's chain sums: 32, and room for reads past them
+struct DevSolo {
+    const void* blk;
+    const SoloLists* lists;     // per wave
+    const int2* cls_draw;       // per class: {first position, draws made ahead}
+    const SoloWide* wide;       // in class order
+    int n_wide;
+    int wide_chains;            // the longest wide bit's chains
+};
+size_t solo_dynamic_lds(int n, int n_rays, int wide_chains, int precision, bool bits);
+size_t solo_lds_limit();
+hipError_t launch_solo_blocks(const DevProblem& p, const SoloTile* tiles, const SlotDesc* desc, int n_tiles, void* blk,
+                              SoloWide* wide, int n_wide, hipStream_t st);
+// Branches 0 .. R - 1, one workgroup each: x (R x n, u16, bit 0) and r (R x n_rays) receive
+// the state after sweep_end, and hold it on entry when sweep_begin > 0.
+hipError_t launch_ray_solo(const DevProblem& p, const DevSolo& d, int precision, void* x, void* r, int R,
+                           uint64_t seed_offset, const double* beta, int sweep_begin, int sweep_end,
+                           int recompute_every, hipStream_t st);
+
 // ---- launchers (qb_kernels.hip) ----
 // Writes every packed batch's block (DevBatches::blk) from its slot descriptors.
 hipError_t launch_batch_blocks(const DevProblem& p, const SlotDesc* desc, const int2* meta, int n_batches, int slots,
@@ -375,6 +431,16 @@ __device__ __forceinline__ unsigned xcc_id() { return __builtin_amdgcn_s_getreg(
 template <typename V>
 __device__ __forceinline__ V ld_l2(const V* p) {
     return __hip_atomic_load(const_cast<V*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ T residual_add(T r, float a, double delta);
+template <>
+__device__ __forceinline__ double residual_add<double>(double r, float a, double delta) {
+    return r + double(a) * delta;                       // r[ray] += a * delta (ising_recon.hpp:139)
+}
+template <>
+__device__ __forceinline__ float residual_add<float>(float r, float a, double delta) {
+    return r + (delta > 0.0 ? a : -a);                  // the FP32 carry: one float add
 }
 #endif
 

@@ -68,17 +68,6 @@ __device__ __forceinline__ bool grid_barrier(unsigned* bar, unsigned target, int
     return s_ok != 0;
 }
 
-template <typename T>
-__device__ __forceinline__ T residual_add(T r, float a, double delta);
-template <>
-__device__ __forceinline__ double residual_add<double>(double r, float a, double delta) {
-    return r + double(a) * delta;                       // r[ray] += a * delta (ising_recon.hpp:139)
-}
-template <>
-__device__ __forceinline__ float residual_add<float>(float r, float a, double delta) {
-    return r + (delta > 0.0 ? a : -a);                  // the FP32 carry: one float add
-}
-
 // ---------------------------------------------------------------------------------
 // XCD teams. The sweep's workgroups form one team per XCD (the hardware XCC_ID), and
 // a team anneals its own branch groups alone. Inside an XCD the L2 is the point of
@@ -1619,6 +1608,12 @@ int ray_energy_blocks(const DevProblem& p, int bw) {
     return (p.n_rays + items - 1) / items + (p.n + items - 1) / items;
 }
 
+// The energy kernels also take width 1 (one branch per group, the small problems' layout).
+template <typename F>
+static hipError_t with_energy_bw(int bw, F&& fn) {
+    return bw == 1 ? fn.template operator()<1>() : with_bw(bw, fn);
+}
+
 hipError_t launch_ray_energy(const DevProblem& p, const uint16_t* x, int n_groups, int bw, int R, const void* r_carried,
                              int precision, double* part, int n_part_blocks, double* data, double* prior,
                              float* resid_err, hipStream_t st, double* total) {
@@ -1628,7 +1623,7 @@ hipError_t launch_ray_energy(const DevProblem& p, const uint16_t* x, int n_group
     if (bd + bp > n_part_blocks) return hipErrorInvalidValue;
     const int stride = n_groups * bw;
     double* part_prior = part + size_t(bd) * stride;
-    return with_bw(bw, [&]<int BW>() {
+    return with_energy_bw(bw, [&]<int BW>() {
         if (bd > 0) {
             const dim3 grid{unsigned(bd), unsigned(n_groups), 1u};
             if (precision == 1)
