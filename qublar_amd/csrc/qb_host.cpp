@@ -321,7 +321,7 @@ struct qb_problem {
     std::unique_ptr<Solo> solo;   // the one-workgroup-per-branch plan, made on first use
     double solo_us = -1.0;        // its estimated time per sweep, < 0 until asked for
     // workspace
-    DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_rref,
+    DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_x16, w_rref,
         w_rng, w_energy;
     int device = 0;   // the device current at creation: its stream, buffers and scratch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1106,13 +1106,15 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
             team_size_for(o.workgroups, o.precision, bw, sweep_dynamic_lds(P->n_classes, bw, bt->heavy_lds != 0, o.precision));
         if (checked <= 0) return -checked;
     }
-    const int n_part = ray_energy_blocks(P->dev, bw);
+    const int n_part = ray_energy_blocks(P->dev);
+    const int n16 = (R + kGroup - 1) / kGroup;   // groups of the energy kernels
     if ((rc = P->w_x.reserve(sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
         (rc = P->w_r.reserve(tsz * size_t(n_groups) * size_t(std::max(nr, 1)) * size_t(bw))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
         (rc = P->w_bar.reserve(sizeof(unsigned) * (kBarWords + kTicketWords))) ||
         (rc = P->w_err.reserve(sizeof(int))) ||
-        (rc = P->w_part.reserve(sizeof(double) * size_t(n_part) * size_t(n_groups) * size_t(bw))) ||
+        (rc = P->w_part.reserve(sizeof(double) * size_t(n_part) * size_t(n16) * kGroup)) ||
+        (rc = P->w_x16.reserve(bw == kGroup ? 1 : sizeof(uint16_t) * size_t(n16) * size_t(std::max(n, 1)))) ||
         (rc = P->w_pv.reserve(sizeof(float) * size_t(std::max(n, 1)))) || (rc = P->w_tri.reserve(size_t(std::max(n, 1)))) ||
         (rc = P->w_cert.reserve(sizeof(float) * size_t(std::max(n, 1)))) ||
         (rc = P->w_br.reserve(branches ? size_t(R) * size_t(std::max(n, 1)) : 1)) ||
@@ -1151,9 +1153,13 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
     const bool want_energy = energy || rep;
     if (want_energy) {
         QB_HIP(hipMemsetAsync(P->w_rerr.p, 0, sizeof(float), st));
-        QB_HIP(launch_ray_energy(P->dev, P->w_x.as<uint16_t>(), n_groups, bw, R, P->w_r.p, o.precision,
-                                 P->w_part.as<double>(), n_part, P->w_data.as<double>(), P->w_prior.as<double>(),
-                                 P->w_rerr.as<float>(), st));
+        const uint16_t* x16 = P->w_x.as<uint16_t>();
+        if (bw != kGroup) {
+            QB_HIP(launch_regroup(P->w_x.as<uint16_t>(), n, n_groups, bw, P->w_x16.as<uint16_t>(), st));
+            x16 = P->w_x16.as<uint16_t>();
+        }
+        QB_HIP(launch_ray_energy(P->dev, x16, R, P->w_r.p, bw, o.precision, P->w_part.as<double>(), n_part,
+                                 P->w_data.as<double>(), P->w_prior.as<double>(), P->w_rerr.as<float>(), st));
     }
     if (p_void) QB_HIP(hipMemcpyAsync(p_void, P->w_pv.p, sizeof(float) * size_t(n), hipMemcpyDeviceToHost, st));
     if (tri) QB_HIP(hipMemcpyAsync(tri, P->w_tri.p, size_t(n), hipMemcpyDeviceToHost, st));
@@ -1463,7 +1469,7 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
         per_launch = int(std::clamp(kRefFloatUpdatesPerLaunch / (double(R) * double(std::max(n, 1))), 1.0,
                                     double(std::max(total, 1))));
     const int n_groups = (R + kGroup - 1) / kGroup;
-    const int n_part = ray_energy_blocks(P->dev, kGroup);
+    const int n_part = ray_energy_blocks(P->dev);
     if ((rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
         (rc = P->w_rref.reserve(sizeof(double) * size_t(R) * size_t(std::max(nr, 1)))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
@@ -1499,7 +1505,7 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
                                   branches ? P->w_br.as<uint8_t>() : nullptr, st));
     const bool want_energy = energy != nullptr;
     if (want_energy)
-        QB_HIP(launch_ray_energy(P->dev, P->w_x.as<uint16_t>(), n_groups, kGroup, R, nullptr, 0, P->w_part.as<double>(),
+        QB_HIP(launch_ray_energy(P->dev, P->w_x.as<uint16_t>(), R, nullptr, kGroup, 0, P->w_part.as<double>(),
                                  n_part, P->w_data.as<double>(), P->w_prior.as<double>(), nullptr, st));
     if (p_void) QB_HIP(hipMemcpyAsync(p_void, P->w_pv.p, sizeof(float) * size_t(n), hipMemcpyDeviceToHost, st));
     if (tri) QB_HIP(hipMemcpyAsync(tri, P->w_tri.p, size_t(n), hipMemcpyDeviceToHost, st));
@@ -1576,7 +1582,7 @@ static EnergyWorkspace energy_workspace(const qb_problem* P, int K) {
     EnergyWorkspace L;
     const size_t n = size_t(std::max(P->n, 1));
     L.n_groups = (K + kGroup - 1) / kGroup;
-    L.n_part = ray_energy_blocks(P->dev, kGroup);
+    L.n_part = ray_energy_blocks(P->dev);
     L.X = 0;
     L.x = L.X + up(size_t(K) * n);
     L.part = L.x + up(sizeof(uint16_t) * size_t(L.n_groups) * n);
@@ -1598,7 +1604,7 @@ static int energy_into(qb_problem* P, const uint8_t* X, int K, unsigned char* ws
         QB_HIP(hipMemcpyAsync(at(L.X), X, size_t(K) * size_t(n), hipMemcpyHostToDevice, st));
         QB_HIP(launch_pack_states(at(L.X), K, n, P->dev.pos_bit, reinterpret_cast<uint16_t*>(at(L.x)), st));
     }
-    QB_HIP(launch_ray_energy(P->dev, reinterpret_cast<const uint16_t*>(at(L.x)), L.n_groups, kGroup, K, nullptr, 0,
+    QB_HIP(launch_ray_energy(P->dev, reinterpret_cast<const uint16_t*>(at(L.x)), K, nullptr, kGroup, 0,
                              reinterpret_cast<double*>(at(L.part)), L.n_part, reinterpret_cast<double*>(at(L.data)),
                              reinterpret_cast<double*>(at(L.prior)), nullptr, st,
                              reinterpret_cast<double*>(at(L.total))));

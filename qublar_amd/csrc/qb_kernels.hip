@@ -1317,51 +1317,81 @@ __global__ void ray_outputs_kernel(DevProblem p, const uint16_t* x, int n_groups
 // ---- FP64 energies -------------------------------------------------------------------
 constexpr int kEnergyBlock = 256;
 
+// The energy kernels read the branches in groups of kGroup, so that an entry or a neighbour
+// is read once for 16 branches whatever the anneal's group width (at width 2 the data
+// kernel's eight passes over the 39M entries of the gravimetry QUBO took 1.9 ms, this 0.4).
+// Spin masks of width `bw` into masks of kGroup branches.
+__global__ void __launch_bounds__(256) regroup_kernel(const uint16_t* x, int n, int n_groups, int bw, uint16_t* x16) {
+    const int pos = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (pos >= n) return;
+    const int per = kGroup / bw;
+    unsigned m = 0;
+    for (int q = 0; q < per; ++q) {
+        const int g = int(blockIdx.y) * per + q;
+        if (g < n_groups) m |= (unsigned(x[size_t(g) * size_t(n) + pos]) & ((1u << bw) - 1u)) << (q * bw);
+    }
+    x16[size_t(blockIdx.y) * size_t(n) + pos] = uint16_t(m);
+}
+
 // Data term per (ray, branch lane): 1/2 w r^2 with r from scratch, summed over the
-// block's rays per lane; also max |r_carried - r_scratch|.
-template <typename T, int BW>
+// block's rays per lane; also max |r_carried - r_scratch| over the R branches, r_carried in
+// groups of bw.
+template <typename T>
 __global__ void __launch_bounds__(kEnergyBlock)
-ray_energy_data_kernel(DevProblem p, const uint16_t* x, const T* r_carried, double* part, int part_stride,
-                       float* resid_err) {
-    constexpr int kItems = kEnergyBlock / BW;
+ray_energy_data_kernel(DevProblem p, const uint16_t* x, const T* r_carried, int bw, int R, double* part,
+                       int part_stride, float* resid_err) {
+    constexpr int kItems = kEnergyBlock / kGroup;
     __shared__ double red[kEnergyBlock];
-    const int b = threadIdx.x % BW;
+    const int b = threadIdx.x % kGroup;
     const int g = blockIdx.y;
-    const int ray = blockIdx.x * kItems + int(threadIdx.x / BW);
+    const int ray = blockIdx.x * kItems + int(threadIdx.x / kGroup);
     double v = 0.0;
     float err = 0.0f;
     if (ray < p.n_rays) {
         const uint16_t* xg = x + size_t(g) * size_t(p.n);
         double r = -p.d[ray];
-        for (int k = p.rt_ptr[ray]; k < p.rt_ptr[ray + 1]; ++k) {
-            const BitEnt e = p.rt[k];
-            if ((xg[e.pos] >> b) & 1) r += double(e.a);
+        const int q0 = p.rt_ptr[ray], q1 = p.rt_ptr[ray + 1];
+        for (int qa = q0; qa < q1; qa += kSeg) {
+            // the chunk's entries, then its spin masks, in flight together; added in order
+            BitEnt e[kSeg];
+            uint16_t m[kSeg];
+#pragma unroll
+            for (int u = 0; u < kSeg; ++u) e[u] = p.rt[min(qa + u, q1 - 1)];
+#pragma unroll
+            for (int u = 0; u < kSeg; ++u) m[u] = xg[e[u].pos];
+#pragma unroll
+            for (int u = 0; u < kSeg; ++u) {
+                const double nxt = r + double(e[u].a);
+                r = (qa + u < q1 && ((m[u] >> b) & 1)) ? nxt : r;
+            }
         }
         v = 0.5 * p.w[ray] * r * r;
-        if (r_carried) {
-            const double rc = double(r_carried[(size_t(g) * size_t(p.n_rays) + size_t(ray)) * BW + b]);
+        const int branch = g * kGroup + b;
+        if (r_carried && branch < R) {
+            const double rc =
+                double(r_carried[(size_t(branch / bw) * size_t(p.n_rays) + size_t(ray)) * bw + branch % bw]);
             err = float(fabs(rc - r));
         }
     }
     red[threadIdx.x] = v;
     if (r_carried && err > 0.0f) atomicMax(reinterpret_cast<unsigned*>(resid_err), __float_as_uint(err));
     __syncthreads();
-    for (int stride = kEnergyBlock / 2; stride >= BW; stride >>= 1) {
+    for (int stride = kEnergyBlock / 2; stride >= kGroup; stride >>= 1) {
         if (int(threadIdx.x) < stride) red[threadIdx.x] += red[threadIdx.x + stride];
         __syncthreads();
     }
-    if (int(threadIdx.x) < BW) part[size_t(blockIdx.x) * part_stride + size_t(g) * BW + threadIdx.x] = red[threadIdx.x];
+    if (int(threadIdx.x) < kGroup)
+        part[size_t(blockIdx.x) * part_stride + size_t(g) * kGroup + threadIdx.x] = red[threadIdx.x];
 }
 
 // Prior term per (position, branch lane): lin x + lambda per unlike neighbour j > i.
-template <int BW>
 __global__ void __launch_bounds__(kEnergyBlock)
 ray_energy_prior_kernel(DevProblem p, const uint16_t* x, double* part, int part_stride) {
-    constexpr int kItems = kEnergyBlock / BW;
+    constexpr int kItems = kEnergyBlock / kGroup;
     __shared__ double red[kEnergyBlock];
-    const int b = threadIdx.x % BW;
+    const int b = threadIdx.x % kGroup;
     const int g = blockIdx.y;
-    const int pos = blockIdx.x * kItems + int(threadIdx.x / BW);
+    const int pos = blockIdx.x * kItems + int(threadIdx.x / kGroup);
     double v = 0.0;
     if (pos < p.n) {
         const uint16_t* xg = x + size_t(g) * size_t(p.n);
@@ -1373,25 +1403,53 @@ ray_energy_prior_kernel(DevProblem p, const uint16_t* x, double* part, int part_
     }
     red[threadIdx.x] = v;
     __syncthreads();
-    for (int stride = kEnergyBlock / 2; stride >= BW; stride >>= 1) {
+    for (int stride = kEnergyBlock / 2; stride >= kGroup; stride >>= 1) {
         if (int(threadIdx.x) < stride) red[threadIdx.x] += red[threadIdx.x + stride];
         __syncthreads();
     }
-    if (int(threadIdx.x) < BW) part[size_t(blockIdx.x) * part_stride + size_t(g) * BW + threadIdx.x] = red[threadIdx.x];
+    if (int(threadIdx.x) < kGroup)
+        part[size_t(blockIdx.x) * part_stride + size_t(g) * kGroup + threadIdx.x] = red[threadIdx.x];
 }
 
-// Sums the partials of each branch in block order (deterministic).
-__global__ void ray_energy_final_kernel(const double* part_data, int blocks_data, const double* part_prior,
-                                        int blocks_prior, int stride, int R, double* data, double* prior,
-                                        double* total) {
-    const int br = int(blockIdx.x * blockDim.x + threadIdx.x);
-    if (br >= R) return;
-    double d = 0.0, q = 0.0;
-    for (int k = 0; k < blocks_data; ++k) d += part_data[size_t(k) * stride + br];
-    for (int k = 0; k < blocks_prior; ++k) q += part_prior[size_t(k) * stride + br];
-    data[br] = d;
-    prior[br] = q;
-    if (total) total[br] = d + q;
+// Sums the partials of branch blockIdx.x: thread t adds those of blocks t, t + 256, ... in
+// order, then a tree over the threads, so the result depends on the block counts alone.
+// One lane per branch walking its partials in block order took 3.4 ms for the 23,873
+// partials of 16 states of the muon QUBO (one dependent load and addition each).
+__global__ void __launch_bounds__(kEnergyBlock)
+ray_energy_final_kernel(const double* part_data, int blocks_data, const double* part_prior, int blocks_prior, int stride,
+                        double* data, double* prior, double* total) {
+    __shared__ double red[2][kEnergyBlock];
+    const int br = int(blockIdx.x), t = int(threadIdx.x);
+    auto sum = [&](const double* part, int blocks) {
+        double s = 0.0;
+        constexpr int kAhead = 8;
+        for (int k0 = t; k0 < blocks; k0 += kAhead * kEnergyBlock) {
+            double v[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                const int k = k0 + u * kEnergyBlock;
+                v[u] = k < blocks ? part[size_t(k) * stride + br] : 0.0;
+            }
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) s += v[u];
+        }
+        return s;
+    };
+    red[0][t] = sum(part_data, blocks_data);
+    red[1][t] = sum(part_prior, blocks_prior);
+    __syncthreads();
+    for (int w = kEnergyBlock / 2; w > 0; w >>= 1) {
+        if (t < w) {
+            red[0][t] += red[0][t + w];
+            red[1][t] += red[1][t + w];
+        }
+        __syncthreads();
+    }
+    if (t == 0) {
+        data[br] = red[0][0];
+        prior[br] = red[1][0];
+        if (total) total[br] = red[0][0] + red[1][0];
+    }
 }
 
 // K states (original bit order, one byte per bit) into 16-bit group masks.
@@ -1602,44 +1660,43 @@ hipError_t launch_ray_outputs(const DevProblem& p, const uint16_t* x, int n_grou
     return hipGetLastError();
 }
 
-// Partial-sum blocks of the energy kernels at group width bw.
-int ray_energy_blocks(const DevProblem& p, int bw) {
-    const int items = kEnergyBlock / bw;
+// Partial-sum blocks of the energy kernels.
+int ray_energy_blocks(const DevProblem& p) {
+    const int items = kEnergyBlock / kGroup;
     return (p.n_rays + items - 1) / items + (p.n + items - 1) / items;
 }
 
-// The energy kernels also take width 1 (one branch per group, the small problems' layout).
-template <typename F>
-static hipError_t with_energy_bw(int bw, F&& fn) {
-    return bw == 1 ? fn.template operator()<1>() : with_bw(bw, fn);
+hipError_t launch_regroup(const uint16_t* x, int n, int n_groups, int bw, uint16_t* x16, hipStream_t st) {
+    const int n16 = (n_groups * bw + kGroup - 1) / kGroup;
+    if (n > 0)
+        regroup_kernel<<<dim3(unsigned((n + 255) / 256), unsigned(n16)), 256, 0, st>>>(x, n, n_groups, bw, x16);
+    return hipGetLastError();
 }
 
-hipError_t launch_ray_energy(const DevProblem& p, const uint16_t* x, int n_groups, int bw, int R, const void* r_carried,
+hipError_t launch_ray_energy(const DevProblem& p, const uint16_t* x, int R, const void* r_carried, int bw,
                              int precision, double* part, int n_part_blocks, double* data, double* prior,
                              float* resid_err, hipStream_t st, double* total) {
-    const int items = kEnergyBlock / bw;
+    const int items = kEnergyBlock / kGroup;
+    const int n_groups = (R + kGroup - 1) / kGroup;
     const int bd = (p.n_rays + items - 1) / items;
     const int bp = (p.n + items - 1) / items;
     if (bd + bp > n_part_blocks) return hipErrorInvalidValue;
-    const int stride = n_groups * bw;
+    const int stride = n_groups * kGroup;
     double* part_prior = part + size_t(bd) * stride;
-    return with_energy_bw(bw, [&]<int BW>() {
-        if (bd > 0) {
-            const dim3 grid{unsigned(bd), unsigned(n_groups), 1u};
-            if (precision == 1)
-                ray_energy_data_kernel<float, BW><<<grid, kEnergyBlock, 0, st>>>(
-                    p, x, static_cast<const float*>(r_carried), part, stride, resid_err);
-            else
-                ray_energy_data_kernel<double, BW><<<grid, kEnergyBlock, 0, st>>>(
-                    p, x, static_cast<const double*>(r_carried), part, stride, resid_err);
-        }
-        if (bp > 0)
-            ray_energy_prior_kernel<BW><<<dim3(unsigned(bp), unsigned(n_groups)), kEnergyBlock, 0, st>>>(p, x, part_prior,
-                                                                                                      stride);
-        ray_energy_final_kernel<<<unsigned((R + 63) / 64), 64, 0, st>>>(part, bd, part_prior, bp, stride, R, data, prior,
-                                                                              total);
-        return hipGetLastError();
-    });
+    if (bd > 0) {
+        const dim3 grid{unsigned(bd), unsigned(n_groups), 1u};
+        if (precision == 1)
+            ray_energy_data_kernel<float><<<grid, kEnergyBlock, 0, st>>>(p, x, static_cast<const float*>(r_carried), bw,
+                                                                         R, part, stride, resid_err);
+        else
+            ray_energy_data_kernel<double><<<grid, kEnergyBlock, 0, st>>>(p, x, static_cast<const double*>(r_carried),
+                                                                          bw, R, part, stride, resid_err);
+    }
+    if (bp > 0)
+        ray_energy_prior_kernel<<<dim3(unsigned(bp), unsigned(n_groups)), kEnergyBlock, 0, st>>>(p, x, part_prior,
+                                                                                              stride);
+    ray_energy_final_kernel<<<unsigned(R), kEnergyBlock, 0, st>>>(part, bd, part_prior, bp, stride, data, prior, total);
+    return hipGetLastError();
 }
 
 hipError_t launch_pack_states(const uint8_t* X, int K, int n, const int32_t* pos_bit, uint16_t* x, hipStream_t st) {
