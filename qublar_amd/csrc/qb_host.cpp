@@ -2616,92 +2616,79 @@ extern "C" int qb_roi_enumerate(int n, const double* h, const double* J, double 
     if (n < 1 || n > 36) return fail(QB_E_ARG, "qb_roi_enumerate: n = %d, must be 1..36", n);
     if (!h || !J || !out) return fail(QB_E_ARG, "qb_roi_enumerate: null argument");
     if (!(beta >= 0.0) || !std::isfinite(beta)) return fail(QB_E_ARG, "beta must be finite and >= 0");
-    std::vector<double> Js(size_t(n) * size_t(n), 0.0);
+    // smaller problems are padded with free bits (no field, no coupling): they repeat every
+    // state, which leaves the minimum (its smallest index has them unset) and the marginals as
+    // they are and multiplies Z by a power of two
+    const int m = std::max(n, kRoiMinBits);
+    const unsigned blocks = roi_blocks(m);
+    // one buffer, in doubles: the inputs, the results, the partials
+    const size_t at_J = size_t(m), at_f = at_J + size_t(m) * size_t(m);
+    const size_t inputs = at_f + size_t(kRoiGroupBits) * kRoiGroupBits;
+    const size_t at_e = inputs, at_s = at_e + 1, at_out = at_s + 1, results = size_t(m) + 3;
+    const size_t at_blk = at_e + results;   // blk_e and blk_s, then the sums in the same place
+    const size_t bytes = sizeof(double) * (at_blk + size_t(blocks) * size_t(kRoiSums));
+    std::vector<double> in(inputs, 0.0);
     for (int i = 0; i < n; ++i) {
         if (!std::isfinite(h[i])) return fail(QB_E_ARG, "h[%d] is not finite", i);
+        in[size_t(i)] = h[i];
         for (int j = i + 1; j < n; ++j) {
             const double v = J[size_t(i) * size_t(n) + size_t(j)];
             if (!std::isfinite(v)) return fail(QB_E_ARG, "J[%d][%d] is not finite", i, j);
-            Js[size_t(i) * size_t(n) + size_t(j)] = Js[size_t(j) * size_t(n) + size_t(i)] = v;
+            in[at_J + size_t(i) * size_t(m) + size_t(j)] = in[at_J + size_t(j) * size_t(m) + size_t(i)] = v;
         }
     }
-    // 2^k states per thread (k <= 12 keeps the carried energy near a scratch sum), the
-    // chunks split over launches of at most 2^22 threads
-    const int k = std::max(0, std::min(n - 14, 12));
-    const uint64_t chunks = uint64_t(1) << (n - k);
-    const uint64_t per_launch = uint64_t(1) << 22;
-    const int nmax = roi_nmax(n);
-    const size_t max_blocks = size_t((std::min(chunks, per_launch) + 255) / 256);
-    DevBuf d_h, d_J, d_e, d_s, d_m;
+    // the group bits' weights multiply only while no factor can leave a double's range
+    double reach = 0.0;
+    for (int a = 0; a < kRoiGroupBits; ++a) {
+        reach += std::fabs(in[size_t(a)]);
+        for (int j = 0; j < m; ++j) reach += std::fabs(in[at_J + size_t(a) * size_t(m) + size_t(j)]);
+        for (int k = 0; k < a; ++k)
+            in[at_f + size_t(a * kRoiGroupBits + k)] = std::exp(-beta * in[at_J + size_t(a) * size_t(m) + size_t(k)]);
+    }
+    const bool products = beta * reach < 600.0;
+    DevBuf buf;
     int rc;
-    if ((rc = d_h.reserve(sizeof(double) * size_t(n))) || (rc = d_J.reserve(sizeof(double) * Js.size())) ||
-        (rc = d_e.reserve(sizeof(double) * max_blocks)) || (rc = d_s.reserve(sizeof(uint64_t) * max_blocks)) ||
-        (rc = d_m.reserve(sizeof(double) * max_blocks * size_t(nmax + 1))))
-        return rc;
-    QB_HIP(hipMemcpy(d_h.p, h, sizeof(double) * size_t(n), hipMemcpyHostToDevice));
-    QB_HIP(hipMemcpy(d_J.p, Js.data(), sizeof(double) * Js.size(), hipMemcpyHostToDevice));
-    hipEvent_t e0, e1;
-    QB_HIP(hipEventCreate(&e0));
-    QB_HIP(hipEventCreate(&e1));
+    if ((rc = buf.reserve(bytes))) return rc;
+    double* d = buf.as<double>();
     struct Events {
-        hipEvent_t a, b;
+        hipEvent_t a = nullptr, b = nullptr;
         ~Events() {
-            (void)hipEventDestroy(a);
-            (void)hipEventDestroy(b);
+            if (a) (void)hipEventDestroy(a);
+            if (b) (void)hipEventDestroy(b);
         }
-    } ev{e0, e1};
-    double kernel_ms = 0.0;
-    // pass 1: the minimum energy and its state (ties to the smallest index)
-    double e_min = std::numeric_limits<double>::infinity();
+    } ev;
+    QB_HIP(hipEventCreate(&ev.a));
+    QB_HIP(hipEventCreate(&ev.b));
+    QB_HIP(hipMemcpy(d, in.data(), sizeof(double) * inputs, hipMemcpyHostToDevice));
+    QB_HIP(hipEventRecord(ev.a, nullptr));
+    QB_HIP(launch_roi_min(m, d, d + at_J, d + at_blk, reinterpret_cast<uint64_t*>(d + at_blk + blocks), d + at_e,
+                          reinterpret_cast<uint64_t*>(d + at_s), nullptr));
+    QB_HIP(launch_roi_sum(m, d, d + at_J, beta, d + at_e, d + at_f, products, d + at_blk, d + at_out, nullptr));
+    QB_HIP(hipEventRecord(ev.b, nullptr));
+    std::vector<double> res(results);
+    QB_HIP(hipMemcpy(res.data(), d + at_e, sizeof(double) * results, hipMemcpyDeviceToHost));
+    float ms = 0.0f;
+    QB_HIP(hipEventElapsedTime(&ms, ev.a, ev.b));
     uint64_t s_min = 0;
-    std::vector<double> be(max_blocks);
-    std::vector<uint64_t> bs(max_blocks);
-    for (uint64_t c0 = 0; c0 < chunks; c0 += per_launch) {
-        const uint64_t cn = std::min(per_launch, chunks - c0);
-        const size_t blocks = size_t((cn + 255) / 256);
-        QB_HIP(hipEventRecord(e0, nullptr));
-        QB_HIP(launch_roi_min(n, k, d_h.as<double>(), d_J.as<double>(), c0, cn, d_e.as<double>(), d_s.as<uint64_t>(),
-                              nullptr));
-        QB_HIP(hipEventRecord(e1, nullptr));
-        QB_HIP(hipMemcpy(be.data(), d_e.p, sizeof(double) * blocks, hipMemcpyDeviceToHost));
-        QB_HIP(hipMemcpy(bs.data(), d_s.p, sizeof(uint64_t) * blocks, hipMemcpyDeviceToHost));
-        float ms = 0.0f;
-        QB_HIP(hipEventElapsedTime(&ms, e0, e1));
-        kernel_ms += ms;
-        for (size_t b = 0; b < blocks; ++b)
-            if (be[b] < e_min || (be[b] == e_min && bs[b] < s_min)) {
-                e_min = be[b];
-                s_min = bs[b];
-            }
-    }
-    // pass 2: Z and the weighted bit sums relative to the minimum, reduced in block order
-    double z = 0.0;
-    std::vector<double> msum(size_t(n), 0.0), bm(max_blocks * size_t(nmax + 1));
-    for (uint64_t c0 = 0; c0 < chunks; c0 += per_launch) {
-        const uint64_t cn = std::min(per_launch, chunks - c0);
-        const size_t blocks = size_t((cn + 255) / 256);
-        QB_HIP(hipEventRecord(e0, nullptr));
-        QB_HIP(launch_roi_sum(n, k, d_h.as<double>(), d_J.as<double>(), beta, e_min, c0, cn, d_m.as<double>(), nullptr));
-        QB_HIP(hipEventRecord(e1, nullptr));
-        QB_HIP(hipMemcpy(bm.data(), d_m.p, sizeof(double) * blocks * size_t(nmax + 1), hipMemcpyDeviceToHost));
-        float ms = 0.0f;
-        QB_HIP(hipEventElapsedTime(&ms, e0, e1));
-        kernel_ms += ms;
-        for (size_t b = 0; b < blocks; ++b) {
-            const double* row = bm.data() + b * size_t(nmax + 1);
-            for (int i = 0; i < n; ++i) msum[size_t(i)] += row[i];
-            z += row[nmax];
-        }
+    std::memcpy(&s_min, &res[1], sizeof s_min);
+    const double z = std::ldexp(res[2], n - m);
+    // the minimum state's energy from scratch
+    double e_min = 0.0;
+    for (int i = 0; i < n; ++i) {
+        if (!((s_min >> i) & 1u)) continue;
+        e_min += h[i];
+        for (int j = i + 1; j < n; ++j)
+            if ((s_min >> j) & 1u) e_min += J[size_t(i) * size_t(n) + size_t(j)];
     }
     if (marginal)
-        for (int i = 0; i < n; ++i) marginal[i] = msum[size_t(i)] / z;
+        for (int i = 0; i < n; ++i) marginal[i] = res[size_t(3 + i)] / res[2];
     if (map_state)
         for (int i = 0; i < n; ++i) map_state[i] = uint8_t((s_min >> i) & 1u);
     out->e_min = e_min;
-    out->log_z = -beta * e_min + std::log(z);
+    out->log_z = -beta * res[0] + std::log(z);
     out->p_map = 1.0 / z;
     out->map_index = s_min;
     out->states = std::ldexp(1.0, n);
-    out->kernel_ms = kernel_ms;
+    out->kernel_ms = ms;
     return QB_OK;
 }

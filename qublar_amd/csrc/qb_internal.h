@@ -446,12 +446,23 @@ __device__ __forceinline__ float residual_add<float>(float r, float a, double de
 #endif
 
 // ---- exact region-of-interest posterior (qb_roi.hip) -----------------------------------
-// Couplings symmetric with a zero diagonal (Js, n x n), chunks of 2^k states per thread.
-int roi_nmax(int n);
-hipError_t launch_roi_min(int n, int k, const double* h, const double* Js, uint64_t chunk0, uint64_t chunks,
-                          double* blk_e, uint64_t* blk_s, hipStream_t st);
-// blk: per block NMAX weighted bit sums and Z (roi_nmax(n) + 1 doubles).
-hipError_t launch_roi_sum(int n, int k, const double* h, const double* Js, double beta, double e_ref, uint64_t chunk0,
-                          uint64_t chunks, double* blk, hipStream_t st);
+// The state index from its lowest bit: kRoiGroupBits bits taken 32 states at once, the walked
+// bits, kRoiThreadBits thread bits, block bits. n is at least kRoiMinBits (the host pads
+// smaller problems with free bits). Couplings symmetric with a zero diagonal (Js, n x n).
+constexpr int kRoiGroupBits = 5;
+constexpr int kRoiThreadBits = 8;
+constexpr int kRoiMaxWalked = 7;
+constexpr int kRoiMinBits = kRoiGroupBits + kRoiThreadBits;
+constexpr int kRoiSums = 1 + kRoiGroupBits + kRoiMaxWalked + kRoiThreadBits;   // values of a block's partial sums
+int roi_walked_bits(int n);
+inline unsigned roi_blocks(int n) { return 1u << (n - kRoiGroupBits - roi_walked_bits(n) - kRoiThreadBits); }
+// The minimum energy and its smallest state (blk_e, blk_s: roi_blocks(n) values each).
+hipError_t launch_roi_min(int n, const double* h, const double* Js, double* blk_e, uint64_t* blk_s, double* e_min,
+                          uint64_t* s_min, hipStream_t st);
+// out[0] = Z relative to *e_min, out[1 + i] = bit i's weight (blk: roi_blocks(n) x kRoiSums).
+// factors[a * kRoiGroupBits + k] = exp(-beta J_ak) among the group bits; with `products` the
+// caller vouches that beta times the group bits' largest fields and couplings stays below 600.
+hipError_t launch_roi_sum(int n, const double* h, const double* Js, double beta, const double* e_min,
+                          const double* factors, bool products, double* blk, double* out, hipStream_t st);
 
 }  // namespace qb
