@@ -1676,7 +1676,8 @@ struct qb_graph {
     qb_plan plan{};
     bool lds_state = false;
     std::vector<int32_t> pos_bit, cls_ptr;
-    DevBuf b_cls, b_pos, b_nbp, b_nb, b_nw, b_f0, b_eu, b_ev, b_ew, b_bitpos;
+    DevBuf b_cls, b_pos, b_nbp, b_nb, b_nw, b_f0, b_eu, b_ev, b_ew, b_bitpos, b_orows, b_prows, b_ostart, b_band;
+    int cus = 0;   // compute units of its device
     DevBuf w_s, w_f, w_e, w_sout, w_beta, w_X, w_out, w_rng;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ~qb_graph() {
@@ -1836,6 +1837,36 @@ extern "C" int qb_graph_create(const qb_graph_desc* d, int force_global, qb_grap
     hipStream_t st = G->stream;
     std::vector<int32_t> eu(d->eu, d->eu + m), ev(d->ev, d->ev + m), ewv(d->ew, d->ew + m);
     int rc;
+    hipDeviceProp_t prop;
+    if ((rc = device_props(prop))) return rc;
+    G->cus = prop.multiProcessorCount;
+    // rows of 16-bit words where one magnitude serves every coupling
+    const bool one_weight = n <= 32768 && m > 0 && 2 * m <= int64_t(INT32_MAX) && G->plan.max_w < (int64_t(1) << 30) &&
+                            std::all_of(w.begin(), w.end(), [&](int32_t v) { return v != 0 && std::abs(int64_t(v)) == G->plan.max_w; });
+    if (one_weight) {
+        std::vector<uint16_t> orows(size_t(2 * m)), prows(size_t(2 * m));
+        std::vector<int32_t> ostart(row.begin(), row.end());
+        for (size_t q = 0; q < orows.size(); ++q) {
+            orows[q] = uint16_t(col[q] | (w[q] < 0 ? 0x8000 : 0));
+            prows[q] = uint16_t(nb[q] | (nw[q] < 0 ? 0x8000 : 0));
+        }
+        std::vector<uint64_t> band(static_cast<size_t>(n), 0u);
+        for (int i = 0; i < n; ++i)
+            for (int64_t k = row[size_t(i)]; k < row[size_t(i) + 1]; ++k) {
+                const int back = i - col[size_t(k)];
+                if (back >= 1 && back <= 64) band[size_t(i)] |= uint64_t(1) << (64 - back);
+            }
+        if ((rc = G->b_band.upload(band, st)) || (rc = G->b_orows.upload(orows, st)) || (rc = G->b_prows.upload(prows, st)) ||
+            (rc = G->b_ostart.upload(ostart, st)))
+            return rc;
+        QB_HIP(hipStreamSynchronize(st));
+        G->dev.orows = G->b_orows.as<uint16_t>();
+        G->dev.prows = G->b_prows.as<uint16_t>();
+        G->dev.ostart = G->b_ostart.as<int32_t>();
+        G->dev.band = G->b_band.as<uint64_t>();
+        G->dev.w0 = int(G->plan.max_w);
+        G->dev.m_dir = int(2 * m);
+    }
     if ((rc = G->b_cls.upload(G->cls_ptr, st)) || (rc = G->b_pos.upload(G->pos_bit, st)) ||
         (rc = G->b_nbp.upload(nb_ptr, st)) || (rc = G->b_nb.upload(nb, st)) || (rc = G->b_nw.upload(nw, st)) ||
         (rc = G->b_f0.upload(f0, st)) || (rc = G->b_eu.upload(eu, st)) || (rc = G->b_ev.upload(ev, st)) ||
@@ -1951,11 +1982,18 @@ extern "C" int qb_run_batch_reference(qb_graph* G, const qb_schedule* b, uint64_
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(G->w_beta.p, temp.data(), sizeof(double) * temp.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(G->ev0, st));
+    bool lds_rows = false;
+    const int waves = int_ref_rows_waves(G->dev, R, G->cus, &lds_rows);
     int launches = 0;
     for (int sb = 0; sb < total; sb += chunk) {
-        QB_HIP(launch_int_ref(G->dev, R, seed_base, G->w_beta.as<double>(), sb, std::min(total, sb + chunk),
-                              sb == 0 ? 1 : 0, G->w_s.as<int8_t>(), G->w_f.as<int32_t>(), G->w_rng.as<uint64_t>(),
-                              G->w_e.as<long long>(), st));
+        const int se = std::min(total, sb + chunk), init = sb == 0 ? 1 : 0;
+        if (waves > 0)
+            QB_HIP(launch_int_ref_rows(G->dev, R, waves, lds_rows, seed_base, G->w_beta.as<double>(), sb, se, init,
+                                       G->w_s.as<int8_t>(), G->w_f.as<int32_t>(), G->w_rng.as<uint64_t>(),
+                                       G->w_e.as<long long>(), st));
+        else
+            QB_HIP(launch_int_ref(G->dev, R, seed_base, G->w_beta.as<double>(), sb, se, init, G->w_s.as<int8_t>(),
+                                  G->w_f.as<int32_t>(), G->w_rng.as<uint64_t>(), G->w_e.as<long long>(), st));
         ++launches;
     }
     QB_HIP(hipEventRecord(G->ev1, st));

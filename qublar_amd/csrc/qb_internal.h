@@ -177,6 +177,14 @@ struct DevGraph {
     const int32_t* nw;
     const int32_t* f0;      // fields of the all-zero assignment
     const int32_t* bit_pos; // original bit -> position
+    // Where every coupling has the magnitude w0 and n <= 32768 (null otherwise): the rows as
+    // 16-bit words, neighbour | sign << 15, padded to whole 32-bit words -- orows in original
+    // bit order with its row starts, prows in position order (starts nb_ptr).
+    const uint16_t* orows;
+    const uint16_t* prows;
+    const int32_t* ostart;
+    const uint64_t* band;   // per original bit: which of the 64 bits before it are neighbours (bit 63: the last)
+    int w0, m_dir;          // m_dir: row entries (2 m)
     const int32_t* eu;      // edge list, original indices
     const int32_t* ev;
     const int32_t* ew;
@@ -344,6 +352,12 @@ bool int_ref_in_lds(const DevGraph& g);
 hipError_t launch_int_ref(const DevGraph& g, int R, uint64_t seed_base, const double* temp, int sweep_begin,
                           int sweep_end, int init, int8_t* s_state, int32_t* f_state, uint64_t* rng,
                           long long* energy, hipStream_t st);
+// The same trajectory on 16-bit rows (in LDS or not), `waves` replicas per workgroup
+// (int_ref_rows_waves > 0).
+int int_ref_rows_waves(const DevGraph& g, int R, int cus, bool* lds_rows);
+hipError_t launch_int_ref_rows(const DevGraph& g, int R, int waves, bool lds_rows, uint64_t seed_base,
+                               const double* temp, int sweep_begin, int sweep_end, int init, int8_t* s_state,
+                               int32_t* f_state, uint64_t* rng, long long* energy, hipStream_t st);
 hipError_t launch_int_unpermute(const DevGraph& g, int R, const int8_t* s_state, int8_t* s_out,
                                 hipStream_t st);
 hipError_t launch_int_energies(const DevGraph& g, const uint8_t* X, int K, long long* out, hipStream_t st);

@@ -151,6 +151,33 @@ __device__ __forceinline__ bool uphill_accept(double x, double u) {
     if (!below && !above) [[unlikely]] return u < qexp(x);   // inside the band
     return below;
 }
+
+// splitmix64 as a counter: the k-th draw from state s mixes s + k kGamma.
+constexpr uint64_t kGamma = 0x9E3779B97F4A7C15ull;
+
+__device__ __forceinline__ uint64_t mix64(uint64_t z) {
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+
+// u < exp(-dE / T) for u = u53 2^-53 and dE > 0, with x = -dE / T the host's quotient.
+// A float exponential of xa = dE * (-1 / T) decides outside a band of 2^-14 around it:
+// xa is within 1e-14 of x, and the float exponential's error, the rounding of xa to float
+// included, is below 2e-5 for -79 < xa <= 0. Inside the band, and for the rare u = 0,
+// the exact quotient and the FP64 qexp decide. qexp and the host's libm exp differ by at
+// most an ulp or two, so a decision can differ from the host's only for a u within that
+// distance of the exponential.
+__device__ __forceinline__ bool ref_accept(uint64_t u53, long long dE, double T, double nrT) {
+    const double xa = double(dE) * nrT;
+    const double u = double(u53) * 0x1.0p-53;
+    if (!(xa > -79.0)) return u < qexp(-double(dE) / T);   // only u = 0 can pass below e^-79
+    constexpr double kBand = 0x1.0p-14;
+    const double e = double(__builtin_amdgcn_exp2f(float(xa) * 1.44269504f));
+    if (u < e * (1.0 - kBand)) return true;
+    if (u > e * (1.0 + kBand)) return false;
+    return u < qexp(-double(dE) / T);
+}
 #endif
 
 }  // namespace qb
