@@ -1676,7 +1676,7 @@ struct qb_graph {
     qb_plan plan{};
     bool lds_state = false;
     std::vector<int32_t> pos_bit, cls_ptr;
-    DevBuf b_cls, b_pos, b_nbp, b_nb, b_nw, b_f0, b_eu, b_ev, b_ew, b_bitpos, b_orows, b_prows, b_ostart, b_band;
+    DevBuf b_cls, b_pos, b_nbp, b_nb, b_nw, b_f0, b_eu, b_ev, b_ew, b_bitpos, b_orows, b_prows, b_ostart, b_band, b_steps;
     int cus = 0;   // compute units of its device
     DevBuf w_s, w_f, w_e, w_sout, w_beta, w_X, w_out, w_rng;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -1856,7 +1856,13 @@ extern "C" int qb_graph_create(const qb_graph_desc* d, int force_global, qb_grap
                 const int back = i - col[size_t(k)];
                 if (back >= 1 && back <= 64) band[size_t(i)] |= uint64_t(1) << (64 - back);
             }
-        if ((rc = G->b_band.upload(band, st)) || (rc = G->b_orows.upload(orows, st)) || (rc = G->b_prows.upload(prows, st)) ||
+        std::vector<int32_t> steps{0};   // every class in equal steps
+        for (int c = 0; c < K; ++c) {
+            const int c0 = G->cls_ptr[size_t(c)], size = G->cls_ptr[size_t(c) + 1] - c0;
+            const int parts = (size + kWideDraws - 1) / kWideDraws;
+            for (int q = 1; q <= parts; ++q) steps.push_back(c0 + int(int64_t(size) * q / parts));
+        }
+        if ((rc = G->b_steps.upload(steps, st)) || (rc = G->b_band.upload(band, st)) || (rc = G->b_orows.upload(orows, st)) || (rc = G->b_prows.upload(prows, st)) ||
             (rc = G->b_ostart.upload(ostart, st)))
             return rc;
         QB_HIP(hipStreamSynchronize(st));
@@ -1864,6 +1870,8 @@ extern "C" int qb_graph_create(const qb_graph_desc* d, int force_global, qb_grap
         G->dev.prows = G->b_prows.as<uint16_t>();
         G->dev.ostart = G->b_ostart.as<int32_t>();
         G->dev.band = G->b_band.as<uint64_t>();
+        G->dev.steps = G->b_steps.as<int32_t>();
+        G->dev.n_steps = int(steps.size()) - 1;
         G->dev.w0 = int(G->plan.max_w);
         G->dev.m_dir = int(2 * m);
     }
@@ -1931,11 +1939,20 @@ extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_bas
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(G->w_beta.p, beta.data(), sizeof(double) * beta.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(G->ev0, st));
+    // force_global keeps the state in global memory
+    const IntShape sh = G->lds_state ? int_shape(G->dev, R, G->cus) : IntShape{kIntSweep, 0};
     int launches = 0;
     for (int sb = 0; sb < total; sb += chunk) {
-        QB_HIP(launch_int_sweeps(G->dev, R, seed_base, G->w_beta.as<double>(), sb, std::min(total, sb + chunk),
-                                 sb == 0 ? 1 : 0, G->w_s.as<int8_t>(), G->w_f.as<int32_t>(), G->w_e.as<long long>(),
-                                 G->lds_state, st));
+        const int se = std::min(total, sb + chunk), init = sb == 0 ? 1 : 0;
+        if (sh.kind == kIntWide || sh.kind == kIntWideL2)
+            QB_HIP(launch_int_wide(G->dev, R, sh, seed_base, G->w_beta.as<double>(), sb, se, init, G->w_s.as<int8_t>(),
+                                   G->w_f.as<int32_t>(), G->w_e.as<long long>(), st));
+        else if (sh.kind == kIntRows || sh.kind == kIntRowsL2)
+            QB_HIP(launch_int_rows(G->dev, R, sh, seed_base, G->w_beta.as<double>(), sb, se, init, G->w_s.as<int8_t>(),
+                                   G->w_f.as<int32_t>(), G->w_e.as<long long>(), st));
+        else
+            QB_HIP(launch_int_sweeps(G->dev, R, seed_base, G->w_beta.as<double>(), sb, se, init, G->w_s.as<int8_t>(),
+                                     G->w_f.as<int32_t>(), G->w_e.as<long long>(), G->lds_state, st));
         ++launches;
     }
     QB_HIP(hipEventRecord(G->ev1, st));

@@ -185,6 +185,8 @@ struct DevGraph {
     const int32_t* ostart;
     const uint64_t* band;   // per original bit: which of the 64 bits before it are neighbours (bit 63: the last)
     int w0, m_dir;          // m_dir: row entries (2 m)
+    const int32_t* steps;   // the classes in steps of at most kWideDraws bits: n_steps + 1 positions
+    int n_steps;
     const int32_t* eu;      // edge list, original indices
     const int32_t* ev;
     const int32_t* ew;
@@ -358,6 +360,25 @@ int int_ref_rows_waves(const DevGraph& g, int R, int cus, bool* lds_rows);
 hipError_t launch_int_ref_rows(const DevGraph& g, int R, int waves, bool lds_rows, uint64_t seed_base,
                                const double* temp, int sweep_begin, int sweep_end, int init, int8_t* s_state,
                                int32_t* f_state, uint64_t* rng, long long* energy, hipStream_t st);
+// The colour-class trajectory with a workgroup per replica.
+constexpr int kWideStepWaves = 8;
+constexpr int kWideDrawWaves = 4;
+constexpr int kWideBlock = 64 * (kWideStepWaves + kWideDrawWaves);
+constexpr int kWideDraws = 64 * kWideDrawWaves;   // bits of a step
+// Which kernel runs a colour-class launch: a wave per replica on the 32-bit rows, a workgroup
+// per replica or several one-wave replicas per workgroup on the 16-bit rows (in LDS, in L2).
+enum IntKind { kIntSweep, kIntWide, kIntWideL2, kIntRows, kIntRowsL2 };
+struct IntShape {
+    IntKind kind;
+    int waves;   // replicas per workgroup (kIntRows, kIntRowsL2)
+};
+IntShape int_shape(const DevGraph& g, int R, int cus);
+hipError_t launch_int_wide(const DevGraph& g, int R, const IntShape& sh, uint64_t seed_base, const double* beta,
+                           int sweep_begin, int sweep_end, int init, int8_t* s_state, int32_t* f_state,
+                           long long* energy, hipStream_t st);
+hipError_t launch_int_rows(const DevGraph& g, int R, const IntShape& sh, uint64_t seed_base, const double* beta,
+                           int sweep_begin, int sweep_end, int init, int8_t* s_state, int32_t* f_state,
+                           long long* energy, hipStream_t st);
 hipError_t launch_int_unpermute(const DevGraph& g, int R, const int8_t* s_state, int8_t* s_out,
                                 hipStream_t st);
 hipError_t launch_int_energies(const DevGraph& g, const uint8_t* X, int K, long long* out, hipStream_t st);

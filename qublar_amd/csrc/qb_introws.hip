@@ -4,7 +4,9 @@
 //
 //   int_ref_rows_kernel  the reference's own trajectory (wising::anneal,
 //                        src/ising_weighted.hpp:250-267), a wave per replica, several
-//                        replicas of a workgroup sharing the rows in LDS.
+//                        replicas of a workgroup sharing the rows in LDS;
+//   int_wide_kernel      the colour-class trajectory (qb_run_batch), a workgroup per
+//                        replica, for few replicas.
 #include <algorithm>
 
 #include "qb_internal.h"
@@ -125,7 +127,7 @@ __global__ void __launch_bounds__(1024) int_ref_rows_kernel(DevGraph g, int R, u
             const int row0 = start[at], row1 = start[at + 1];
             // the window's lanes before this one that are neighbours, lane j in bit j
             const uint64_t near = lane > 0 ? band[at] >> (64 - lane) : 0u;
-            const long long dE = valid ? -(long long)si * (long long)fi : 0;
+            const int dE = valid ? -si * fi : 0;   // the plan bounds it
             const bool up = valid && dE > 0;
             const uint64_t m_up = __ballot(up);
             bool acc = valid && dE <= 0;
@@ -210,6 +212,295 @@ hipError_t launch_int_ref_rows(const DevGraph& g, int R, int waves, bool lds_row
     else
         int_ref_rows_kernel<false><<<blocks, threads, lds, st>>>(g, R, seed_base, temp, sweep_begin, sweep_end, init,
                                                                  s_state, f_state, rng, energy);
+    return hipGetLastError();
+}
+
+// ---- the colour-class trajectory, few replicas -----------------------------------------------
+// A workgroup anneals one replica with its spins, fields and (where they fit) rows in LDS. A
+// class is cut into steps of at most kWideDraws bits; in a step each of kWideStepWaves waves
+// decides its share of the bits and sends out its own flips' rows -- LDS atomics, and no bit
+// of a class reads a field that the class changes, so one barrier per step suffices --
+// while the draw waves make the next step's draws. int_sweep_kernel gives a replica one wave,
+// which decides up to 64 bits, draws for them and walks the flips' rows in L2 one after the
+// other: 0.9 us a class at n = 800, degree 48, 18 classes, where this takes 0.36.
+template <bool LDS_ROWS>
+__global__ void __launch_bounds__(kWideBlock) int_wide_kernel(DevGraph g, uint64_t seed_base, const double* beta,
+                                                              int sweep_begin, int sweep_end, int init,
+                                                              int8_t* s_state, int32_t* f_state, long long* energy) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    __shared__ Draw draws[2][kWideDraws];
+    __shared__ long long red[kWideBlock / 64];
+    const int n = g.n, np = g.n_pad, S = g.n_steps;
+    const int tid = int(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int32_t* start = reinterpret_cast<int32_t*>(smem);
+    int2* steps = reinterpret_cast<int2*>(start + ((n + 4) & ~3));   // {first position, past the last}
+    int32_t* f = reinterpret_cast<int32_t*>(steps + ((S + 1) & ~1));
+    uint16_t* bit = reinterpret_cast<uint16_t*>(f + np);
+    uint16_t* lrows = bit + np;
+    int8_t* s = reinterpret_cast<int8_t*>(lrows + (LDS_ROWS ? (g.m_dir + 7) & ~7 : 0));
+    const uint16_t* rows = LDS_ROWS ? lrows : g.prows;
+    const int r = int(blockIdx.x);
+    int8_t* gs = s_state + size_t(r) * size_t(np);
+    int32_t* gf = f_state + size_t(r) * size_t(np);
+    for (int i = tid; i <= n; i += kWideBlock) start[i] = g.nb_ptr[i];
+    for (int i = tid; i < S; i += kWideBlock) steps[i] = int2{g.steps[i], g.steps[i + 1]};
+    for (int i = tid; LDS_ROWS && i < g.m_dir / 2; i += kWideBlock)   // m_dir is even
+        reinterpret_cast<uint32_t*>(lrows)[i] = reinterpret_cast<const uint32_t*>(g.prows)[i];
+    for (int i = tid; i < n; i += kWideBlock) {
+        bit[i] = uint16_t(g.pos_bit[i]);
+        f[i] = init ? g.f0[i] : gf[i];
+        s[i] = init ? int8_t(-1) : gs[i];
+    }
+    __syncthreads();
+    const uint64_t seed = seed_base + uint64_t(r);
+    const bool stepper = wave < kWideStepWaves;
+    const int w2 = 2 * g.w0;
+    const bool quarters = g.m_dir <= 32 * n;
+    const int di = tid - 64 * kWideStepWaves;   // a draw wave's bit in a step
+    auto put_draw = [&](int2 step, int sweep, float temperature, int buf) {
+        const int p = step.x + di;
+        if (p < step.y)
+            draws[buf][di] = make_draw(draw_u01(seed, uint32_t(sweep), uint32_t(bit[p])), temperature);
+    };
+    auto step_at = [&](int k) {
+        const int2 v = steps[k];
+        return int2{__builtin_amdgcn_readfirstlane(v.x), __builtin_amdgcn_readfirstlane(v.y)};
+    };
+    int2 cur = step_at(0), nxt = step_at(S > 1 ? 1 : 0);
+    double bt_next = beta[sweep_begin];
+    float temp_next = float(1.0 / bt_next);
+    if (!stepper) put_draw(cur, sweep_begin, temp_next, 0);
+    __syncthreads();
+    long long dsum = 0;
+    int buf = 0, ahead = S > 2 ? 2 : 0;
+    for (int sweep = sweep_begin; sweep < sweep_end; ++sweep) {
+        const double bt = bt_next;
+        const float temp = temp_next;
+        bt_next = beta[min(sweep + 1, sweep_end - 1)];
+        temp_next = float(1.0 / bt_next);
+        for (int k = 0; k < S; ++k) {
+            const int2 after = steps[ahead];   // read two steps ahead
+            ahead = ahead + 1 < S ? ahead + 1 : 0;
+            if (stepper) {
+                const int p0 = cur.x, p1 = cur.y;
+                const int share = (p1 - p0 + kWideStepWaves - 1) / kWideStepWaves;   // <= 64
+                const int off = wave * share + lane, pos = p0 + off;
+                const bool mine = lane < share && pos < p1;
+                const int at = mine ? pos : p0;
+                const int si = s[at], fi = f[at];
+                const int row0 = start[at], row1 = start[at + 1];
+                Draw dr = draws[buf][mine ? off : 0];
+                asm("" : "+v"(dr.lo), "+v"(dr.hi));   // read with the others, not in the branch below
+                const int dE = -si * fi;   // State::dE, ising_weighted.hpp:209 (the plan bounds it)
+                bool acc = false;
+                if (mine) {
+                    const float ef = float(dE);
+                    const bool below = dE <= 0 || ef < dr.lo, above = ef > dr.hi;
+                    acc = below;
+                    if (!below && !above) [[unlikely]] acc = uphill_accept(-double(dE) * bt, dr.u);
+                }
+                const uint64_t m = __ballot(acc);
+                if (m) {
+                    if (acc) {
+                        dsum += dE;
+                        s[at] = int8_t(-si);
+                    }
+                    rows_add(rows, m, lane, row0, row1, si, w2, f, quarters);
+                }
+            } else {
+                const bool wrap = k + 1 == S;
+                put_draw(nxt, wrap ? sweep + 1 : sweep, wrap ? temp_next : temp, buf ^ 1);
+            }
+            buf ^= 1;
+            cur = nxt;
+            nxt = int2{__builtin_amdgcn_readfirstlane(after.x), __builtin_amdgcn_readfirstlane(after.y)};
+            __syncthreads();
+        }
+    }
+    for (int i = tid; i < n; i += kWideBlock) {
+        gf[i] = f[i];
+        gs[i] = s[i];
+    }
+    for (int o = 32; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o);
+    if (lane == 0) red[wave] = dsum;
+    __syncthreads();
+    if (tid == 0) {
+        long long t = 0;
+        for (int w = 0; w < kWideBlock / 64; ++w) t += red[w];
+        energy[r] = (init ? 0 : energy[r]) + t;
+    }
+}
+
+static size_t wide_lds(const DevGraph& g, bool lds_rows) {
+    return 4 * (size_t((g.n + 4) & ~3) + 2 * size_t((g.n_steps + 1) & ~1) + size_t(g.n_pad)) + 2 * size_t(g.n_pad) +
+           (lds_rows ? 2 * size_t((g.m_dir + 7) & ~7) : 0) + size_t(g.n_pad);
+}
+constexpr size_t kWideStatic = 2 * kWideDraws * sizeof(Draw) + (kWideBlock / 64) * sizeof(long long);
+
+// ---- the colour-class trajectory, many replicas ----------------------------------------------
+// A wave per replica, as in int_sweep_kernel, several of a workgroup sharing the 16-bit rows
+// in LDS, and an uphill move decided through the float exponential's band instead of the
+// FP64 exponential. Nothing is shared between waves after the rows are in. 8,192 replicas x
+// 1,000 sweeps at n = 800, degree 48: 93.7 -> 63.0 ms; the bound is vector issue (the draws).
+template <bool LDS_ROWS>
+__global__ void __launch_bounds__(1024) int_sweep_rows_kernel(DevGraph g, int R, uint64_t seed_base, const double* beta,
+                                                              int sweep_begin, int sweep_end, int init,
+                                                              int8_t* s_state, int32_t* f_state, long long* energy) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int n = g.n, np = g.n_pad, K = g.n_classes;
+    const int tid = int(threadIdx.x), lane = tid & 63, wave = tid >> 6, block = int(blockDim.x), waves = block / 64;
+    int32_t* start = reinterpret_cast<int32_t*>(smem);
+    int32_t* cls = start + ((n + 4) & ~3);
+    int32_t* fields = cls + ((K + 4) & ~3);
+    uint16_t* bit = reinterpret_cast<uint16_t*>(fields + size_t(waves) * np);
+    uint16_t* lrows = bit + np;
+    int8_t* spins = reinterpret_cast<int8_t*>(lrows + (LDS_ROWS ? (g.m_dir + 7) & ~7 : 0));
+    const uint16_t* rows = LDS_ROWS ? lrows : g.prows;
+    for (int i = tid; i <= n; i += block) start[i] = g.nb_ptr[i];
+    for (int i = tid; i <= K; i += block) cls[i] = g.cls_ptr[i];
+    for (int i = tid; i < n; i += block) bit[i] = uint16_t(g.pos_bit[i]);
+    for (int i = tid; LDS_ROWS && i < g.m_dir / 2; i += block)   // m_dir is even
+        reinterpret_cast<uint32_t*>(lrows)[i] = reinterpret_cast<const uint32_t*>(g.prows)[i];
+    __syncthreads();
+    const int r = int(blockIdx.x) * waves + wave;
+    if (r >= R) return;   // the whole wave leaves; the rest never syncs across waves
+    int32_t* f = fields + size_t(wave) * np;
+    int8_t* s = spins + size_t(wave) * np;
+    int8_t* gs = s_state + size_t(r) * size_t(np);
+    int32_t* gf = f_state + size_t(r) * size_t(np);
+    for (int i = lane; i < n; i += 64) {
+        f[i] = init ? g.f0[i] : gf[i];
+        s[i] = init ? int8_t(-1) : gs[i];
+    }
+    auto sync = [] {
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    sync();
+    const uint64_t seed = seed_base + uint64_t(r);
+    const int w2 = 2 * g.w0;
+    const bool quarters = g.m_dir <= 32 * n;
+    long long dsum = 0;
+    for (int sweep = sweep_begin; sweep < sweep_end; ++sweep) {
+        const double bt = beta[sweep];
+        for (int c = 0; c < K; ++c) {
+            const int c1 = cls[c + 1];
+            for (int base = cls[c]; base < c1; base += 64) {
+                const int pos = base + lane;
+                const bool mine = pos < c1;
+                const int at = mine ? pos : base;
+                const int si = s[at];
+                const int dE = -si * f[at];   // State::dE, ising_weighted.hpp:209 (the plan bounds it)
+                const int row0 = start[at], row1 = start[at + 1];
+                const uint32_t b = bit[at];
+                bool acc = mine && dE <= 0;
+                if (mine && dE > 0) acc = uphill_accept(-double(dE) * bt, draw_u01(seed, uint32_t(sweep), b));
+                const uint64_t m = __ballot(acc);
+                if (m) {
+                    if (acc) {
+                        dsum += dE;
+                        s[at] = int8_t(-si);
+                    }
+                    rows_add(rows, m, lane, row0, row1, si, w2, f, quarters);
+                    sync();
+                }
+            }
+        }
+    }
+    for (int i = lane; i < n; i += 64) {
+        gf[i] = f[i];
+        gs[i] = s[i];
+    }
+    for (int o = 32; o > 0; o >>= 1) dsum += __shfl_xor(dsum, o);
+    if (lane == 0) energy[r] = (init ? 0 : energy[r]) + dsum;
+}
+
+static size_t sweep_rows_lds(const DevGraph& g, int waves, bool lds_rows) {
+    return 4 * (size_t((g.n + 4) & ~3) + size_t((g.n_classes + 4) & ~3)) + 2 * size_t(g.n_pad) +
+           (lds_rows ? 2 * size_t((g.m_dir + 7) & ~7) : 0) + size_t(waves) * g.n_pad * 5;
+}
+
+// The kernel of a colour-class launch of R replicas: the least of the estimated times of a
+// sweep, in us, over the rounds that R takes at what the LDS holds per CU. At one replica a
+// sweep takes about 0.35 per class + 0.045 per bit in int_sweep_kernel, 0.33 per 64 bits of a
+// class + 0.017 per bit in int_sweep_rows_kernel (1.28 times that with the rows in L2), and
+// 0.4 per step + 0.0035 per bit in int_wide_kernel; more waves per CU lengthen it by 4 to
+// 5.5% each, a second int_wide_kernel workgroup by 30%. Measured at n = 100 to 8,000, degree 8
+// to 48 (n = 800, degree 48: 37, 19.5 and 10.3 us at one replica, 42, 21 and 42 at 1,024, 97
+// and 65 at 8,192).
+IntShape int_shape(const DevGraph& g, int R, int cus) {
+    IntShape best{kIntSweep, 0};
+    if (!g.prows) return best;
+    const int per_cu = (R + cus - 1) / cus;
+    auto cost = [&](int capacity, double base, double slope) {
+        const int rounds = (per_cu + capacity - 1) / capacity;
+        return rounds * base * (1.0 + slope * ((per_cu + rounds - 1) / rounds - 1));
+    };
+    const int held = int(std::min<size_t>(32, kRefLdsLimit / (size_t(g.n_pad) * 5)));
+    if (held < 1) return best;
+    double least = 0.95 * cost(held, 0.35 * g.n_classes + 0.045 * g.n, 0.04);
+    for (const bool in_lds : {true, false}) {
+        const double far = in_lds ? 1.0 : 1.28;
+        const size_t wide = wide_lds(g, in_lds) + kWideStatic;
+        if (wide <= kRefLdsLimit) {
+            const int capacity = 2 * wide <= kRefLdsLimit ? 2 : 1;
+            const double c = cost(capacity, 0.4 * g.n_steps + 0.0035 * g.n, 0.3);
+            if (c < least) {
+                least = c;
+                best = IntShape{in_lds ? kIntWide : kIntWideL2, 0};
+            }
+        }
+        int fit = std::min(16, per_cu);
+        while (fit > 0 && sweep_rows_lds(g, fit, in_lds) > kRefLdsLimit) --fit;
+        if (fit > 0) {
+            const int groups = std::max(1, std::min(32 / fit, int(kRefLdsLimit / sweep_rows_lds(g, fit, in_lds))));
+            const double c = cost(fit * groups, far * (0.33 * (g.n / 64.0 + 0.5 * g.n_classes) + 0.017 * g.n),
+                                  in_lds ? 0.04 : 0.055);
+            if (c < least) {
+                least = c;
+                const int rounds = (per_cu + fit - 1) / fit;   // of workgroups
+                best = IntShape{in_lds ? kIntRows : kIntRowsL2, (per_cu + rounds - 1) / rounds};
+            }
+        }
+        if (wide <= kRefLdsLimit) break;   // with the rows in LDS there is no need to ask for L2
+    }
+    return best;
+}
+
+hipError_t launch_int_rows(const DevGraph& g, int R, const IntShape& sh, uint64_t seed_base, const double* beta,
+                           int sweep_begin, int sweep_end, int init, int8_t* s_state, int32_t* f_state,
+                           long long* energy, hipStream_t st) {
+    const bool lds_rows = sh.kind == kIntRows;
+    const size_t lds = sweep_rows_lds(g, sh.waves, lds_rows);
+    const void* k = lds_rows ? reinterpret_cast<const void*>(&int_sweep_rows_kernel<true>)
+                             : reinterpret_cast<const void*>(&int_sweep_rows_kernel<false>);
+    const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+    const unsigned blocks = unsigned((R + sh.waves - 1) / sh.waves), threads = unsigned(64 * sh.waves);
+    if (lds_rows)
+        int_sweep_rows_kernel<true><<<blocks, threads, lds, st>>>(g, R, seed_base, beta, sweep_begin, sweep_end, init,
+                                                                  s_state, f_state, energy);
+    else
+        int_sweep_rows_kernel<false><<<blocks, threads, lds, st>>>(g, R, seed_base, beta, sweep_begin, sweep_end, init,
+                                                                   s_state, f_state, energy);
+    return hipGetLastError();
+}
+
+hipError_t launch_int_wide(const DevGraph& g, int R, const IntShape& sh, uint64_t seed_base, const double* beta, int sweep_begin,
+                           int sweep_end, int init, int8_t* s_state, int32_t* f_state, long long* energy,
+                           hipStream_t st) {
+    const bool lds_rows = sh.kind == kIntWide;
+    const size_t lds = wide_lds(g, lds_rows);
+    const void* k = lds_rows ? reinterpret_cast<const void*>(&int_wide_kernel<true>)
+                             : reinterpret_cast<const void*>(&int_wide_kernel<false>);
+    const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+    if (lds_rows)
+        int_wide_kernel<true><<<unsigned(R), kWideBlock, lds, st>>>(g, seed_base, beta, sweep_begin, sweep_end, init,
+                                                                   s_state, f_state, energy);
+    else
+        int_wide_kernel<false><<<unsigned(R), kWideBlock, lds, st>>>(g, seed_base, beta, sweep_begin, sweep_end, init,
+                                                                    s_state, f_state, energy);
     return hipGetLastError();
 }
 

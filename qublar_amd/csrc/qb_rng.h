@@ -152,6 +152,27 @@ __device__ __forceinline__ bool uphill_accept(double x, double u) {
     return below;
 }
 
+// A draw u as its decision: an uphill move of energy dE (dE beta < 37 wherever it matters)
+// is accepted below lo and refused above hi, and between them u < qexp(-dE beta) decides.
+// lo and hi are (-ln u -+ 2^-14) / beta in float: float(u), log2 and the products are within
+// 2e-5 of the exact exponent together with float(dE), so outside the band the decision is
+// qexp's, bit for bit (uphill_accept's band, written with the logarithm). A zero draw, or a
+// temperature floats cannot hold with room, leaves every uphill move to qexp.
+struct Draw {
+    float lo, hi;
+    double u;
+};
+__device__ __forceinline__ Draw make_draw(double u, float temperature) {
+    constexpr float kBand = 0x1.0p-14f;
+    const float L = -__builtin_amdgcn_logf(float(u)) * 0.69314718f;
+    Draw d{(L - kBand) * temperature, (L + kBand) * temperature, u};
+    if (!(u > 0.0) || !(temperature > 1e-30f) || !(temperature < 1e30f)) {
+        d.lo = 0.0f;
+        d.hi = __builtin_huge_valf();
+    }
+    return d;
+}
+
 // splitmix64 as a counter: the k-th draw from state s mixes s + k kGamma.
 constexpr uint64_t kGamma = 0x9E3779B97F4A7C15ull;
 
@@ -168,7 +189,8 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 // the exact quotient and the FP64 qexp decide. qexp and the host's libm exp differ by at
 // most an ulp or two, so a decision can differ from the host's only for a u within that
 // distance of the exponential.
-__device__ __forceinline__ bool ref_accept(uint64_t u53, long long dE, double T, double nrT) {
+template <typename I>
+__device__ __forceinline__ bool ref_accept(uint64_t u53, I dE, double T, double nrT) {
     const double xa = double(dE) * nrT;
     const double u = double(u53) * 0x1.0p-53;
     if (!(xa > -79.0)) return u < qexp(-double(dE) / T);   // only u = 0 can pass below e^-79

@@ -67,27 +67,6 @@ __device__ __forceinline__ double dpp_double(double v) {
     return u64_double(lo, hi);
 }
 
-// A draw u as its decision: an uphill move of energy dE (dE beta < 37 wherever it matters)
-// is accepted below lo and refused above hi, and between them u < qexp(-dE beta) decides.
-// lo and hi are (-ln u -+ 2^-14) / beta in float: float(u), log2 and the products are within
-// 2e-5 of the exact exponent together with float(dE), so outside the band the decision is
-// qexp's, bit for bit (uphill_accept's band, written with the logarithm). A zero draw, or a
-// temperature floats cannot hold with room, leaves every uphill move to qexp.
-struct Draw {
-    float lo, hi;
-    double u;
-};
-__device__ __forceinline__ Draw make_draw(double u, float temperature) {
-    constexpr float kBand = 0x1.0p-14f;
-    const float L = -__builtin_amdgcn_logf(float(u)) * 0.69314718f;
-    Draw d{(L - kBand) * temperature, (L + kBand) * temperature, u};
-    if (!(u > 0.0) || !(temperature > 1e-30f) || !(temperature < 1e30f)) {
-        d.lo = 0.0f;
-        d.hi = __builtin_huge_valf();
-    }
-    return d;
-}
-
 // A branch's spins in LDS, in position order: a byte per bit where they fit beside the
 // residuals (one instruction fewer per word and shift on each of a bit's seven reads), else
 // a bit.

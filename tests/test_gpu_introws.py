@@ -46,3 +46,29 @@ def test_reference_trajectory_many_replicas(gpu):
     for r in list(range(0, 1037, 61)) + [1034, 1035, 1036]:
         x, en = orc_mod.anneal_int(og, orc_mod.schedule(3.0, 0.2, 12, 3), 1 + r)
         assert np.array_equal((s[r, :g.n] > 0).astype(np.uint8), x) and e[r] == en
+
+
+# the colour-class sweep: a workgroup per replica (classes of fewer bits than step waves, of
+# more than a step holds, rows in L2), then several one-wave replicas per workgroup
+@pytest.mark.parametrize("n,degree,weight", GRAPHS + [(2600, 3, 2)])
+def test_colour_sweep_few_replicas(gpu, n, degree, weight):
+    g = graph(n, degree, weight, signed=n % 2 == 0)
+    if g.m == 0:
+        g = qa.GraphArrays(2, [0], [1], [weight])
+    sched = qa.schedule(weight * max(1.0, degree) ** 0.5, 0.2 * weight, 20, 4)
+    check_int_batch(g, sched, 5, 3)
+    check_int_batch(g, sched, 5, 3, updates_per_launch=5 * g.n * 7)
+
+
+@pytest.mark.parametrize("n,degree,R", [(70, 69, 700), (150, 8, 1300), (600, 40, 1030), (900, 200, 520)])
+def test_colour_sweep_many_replicas(gpu, n, degree, R):
+    g = graph(n, degree, 3)
+    check_int_batch(g, qa.schedule(3.0 * degree ** 0.5, 0.6, 6, 2), R, 11, updates_per_launch=R * n * 5)
+
+
+def test_temperatures_outside_a_float(gpu):
+    """Draws made ahead are bounded in float; temperatures past its range leave every uphill
+    move to the FP64 exponential."""
+    g = graph(90, 10)
+    for t in (1e35, 1e-35):
+        check_int_batch(g, qa.schedule(t, t, 6, 0), 3)
