@@ -305,7 +305,7 @@ struct qb_problem {
     int64_t device_bytes = 0;
     std::vector<int32_t> pos_bit, cls_ptr;
     DevBuf b_cls, b_pos, b_col, b_ent, b_nbp, b_nb, b_nbbit, b_lin, b_d, b_w, b_rtp, b_rt, b_seq, b_dbit, b_dkey,
-        b_lbeg, b_lnb, b_bitpos;
+        b_lbeg, b_lnb, b_bitpos, b_refst;
     std::vector<int32_t> light_begin;   // host copy: each class's first light position
     std::vector<int32_t> col_ptr, nb_ptr;   // host copies, position space
     std::vector<uint8_t> seq_update;
@@ -322,7 +322,8 @@ struct qb_problem {
     double solo_us = -1.0;        // its estimated time per sweep, < 0 until asked for
     // workspace
     DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_x16, w_rref,
-        w_rng, w_energy;
+        w_ref, w_rng, w_energy;
+    size_t ref_entries = 0;   // of the bit-order layout, gaps and padding included
     int device = 0;   // the device current at creation: its stream, buffers and scratch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ~qb_problem() {
@@ -574,6 +575,12 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
     std::vector<BitEnt> rt(static_cast<size_t>(nnz));
     for (size_t q = 0; q < rt.size(); ++q) rt[q] = BitEnt{pos_of[size_t(rt_bit[q])], rt_a[q]};
     std::vector<double> dv(desc->d, desc->d + nr), wv(desc->w, desc->w + nr);
+    std::vector<uint64_t> ref_start(size_t(n) + 1, 0);
+    for (int i = 0; i < n; ++i) {
+        const uint64_t end = ref_start[size_t(i)] + uint64_t(desc->row_ptr[i + 1] - desc->row_ptr[i]);
+        ref_start[size_t(i) + 1] = (i + 1) % 64 == 0 || i + 1 == n ? (end + 255u) & ~uint64_t(255) : end;
+    }
+    P->ref_entries = size_t(ref_start.back()) + kRefPad;
 
     QB_HIP(hipGetDevice(&P->device));
     QB_HIP(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking));
@@ -587,7 +594,8 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
         (rc = P->b_col.upload(col_ptr, st)) || (rc = P->b_ent.upload(ent, st)) || (rc = P->b_nbp.upload(nb_ptr, st)) ||
         (rc = P->b_nb.upload(nb, st)) || (rc = P->b_nbbit.upload(nb_bit, st)) || (rc = P->b_lin.upload(lin, st)) ||
         (rc = P->b_d.upload(dv, st)) || (rc = P->b_w.upload(wv, st)) || (rc = P->b_rtp.upload(rt_ptr, st)) ||
-        (rc = P->b_rt.upload(rt, st)) || (rc = P->b_bitpos.upload(pos_of, st)))
+        (rc = P->b_rt.upload(rt, st)) || (rc = P->b_bitpos.upload(pos_of, st)) ||
+        (rc = P->b_refst.upload(ref_start, st)))
         return rc;
     QB_HIP(hipStreamSynchronize(st));
     P->col_ptr = col_ptr;
@@ -615,6 +623,7 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
     D.bit_pos = P->b_bitpos.as<int32_t>();
     D.col_ptr = P->b_col.as<int32_t>();
     D.ent = P->b_ent.as<RayEnt>();
+    D.ref_start = P->b_refst.as<uint64_t>();
     D.nb_ptr = P->b_nbp.as<int32_t>();
     D.nb = P->b_nb.as<int32_t>();
     D.nb_bit = P->b_nbbit.as<int32_t>();
@@ -1469,8 +1478,12 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
         per_launch = int(std::clamp(kRefFloatUpdatesPerLaunch / (double(R) * double(std::max(n, 1))), 1.0,
                                     double(std::max(total, 1))));
     const int n_groups = (R + kGroup - 1) / kGroup;
+    const size_t n_ref = P->ref_entries;
+    const size_t per_entry = sizeof(double) + sizeof(uint32_t) + sizeof(float) + 1;
+    const size_t per_bit = sizeof(RefBit) + sizeof(RefBase) + sizeof(int32_t) * kRefNb;
     const int n_part = ray_energy_blocks(P->dev);
     if ((rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
+        (rc = P->w_ref.reserve(per_entry * n_ref + per_bit * size_t(n))) ||
         (rc = P->w_rref.reserve(sizeof(double) * size_t(R) * size_t(std::max(nr, 1)))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
         (rc = P->w_x.reserve(sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
@@ -1492,6 +1505,19 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(P->w_beta.p, temp.data(), sizeof(double) * temp.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(P->ev0, st));
+    if (!P->dev.ref.w) {
+        char* at = P->w_ref.as<char>();
+        RefLayout to;
+        to.w = reinterpret_cast<double*>(at);
+        to.bit = reinterpret_cast<RefBit*>(at += sizeof(double) * n_ref);
+        to.base = reinterpret_cast<RefBase*>(at += sizeof(RefBit) * size_t(n));
+        to.nb = reinterpret_cast<int32_t*>(at += sizeof(RefBase) * size_t(n));
+        to.ray = reinterpret_cast<uint32_t*>(at += sizeof(int32_t) * kRefNb * size_t(n));
+        to.a = reinterpret_cast<float*>(at += sizeof(uint32_t) * n_ref);
+        to.own = reinterpret_cast<uint8_t*>(at + sizeof(float) * n_ref);
+        QB_HIP(launch_ref_layout(P->dev, to, n_ref, st));
+        P->dev.ref = to;
+    }
     int launches = 0;
     for (int s0 = 0; s0 < total || launches == 0; s0 += per_launch, ++launches)
         QB_HIP(launch_ray_ref(P->dev, R, seed_offset, P->w_beta.as<double>(), s0, std::min(total, s0 + per_launch),

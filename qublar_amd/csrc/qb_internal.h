@@ -38,6 +38,33 @@ struct BitEnt {
 
 // The float problem on the device, in colour-class position order: position p
 // holds original bit pos_bit[p]; class c is positions [cls_ptr[c], cls_ptr[c+1]).
+// The problem in bit order, as the reference's own trajectory walks it: a window is 64
+// consecutive bits. The entries lie column after column, a window's first at a multiple of
+// 256 (zeros fill the gaps), each with its bit modulo 64; in a block of 256 entries, k lies at
+// ref_slot(k), so that a lane's four consecutive words are entries 64 apart.
+__host__ __device__ inline uint64_t ref_slot(uint64_t k) {
+    return (k & ~uint64_t(255)) | ((k & 63u) << 2) | ((k >> 6) & 3u);
+}
+struct RefBit {
+    uint32_t c0, c1;   // the column's entries, from the window's first
+    uint32_t nb;       // neighbours; top bit: a ray repeats in the column
+    uint32_t q0;       // the first in nb_bit
+};
+struct RefBase {
+    double lin;
+    uint64_t base;   // the window's first entry
+};
+struct RefLayout {
+    double* w;
+    RefBit* bit;
+    RefBase* base;
+    int32_t* nb;   // kRefNb per bit, the bit itself past its last neighbour
+    uint32_t* ray;
+    float* a;
+    uint8_t* own;
+};
+constexpr int kRefNb = 8;
+
 struct DevProblem {
     int n, n_rays, n_classes;
     int64_t nnz, n_nbr;
@@ -62,9 +89,13 @@ struct DevProblem {
     // CSR order (-1 past its last).
     const int32_t* light_begin;
     const int32_t* light_nb;
+    const uint64_t* ref_start;   // the first entry of each bit in ref, and behind the last bit
+    RefLayout ref;               // laid out on the first anneal on the reference's own trajectory
     double lambda;
 };
 constexpr int kLightNb = 8;
+// Zeros after the last entry of RefLayout, so that loads of whole batches may run past it.
+constexpr int kRefPad = 2048;
 
 // Work batches of one sweep step at one group width: a workgroup of BLOCK threads
 // has BLOCK / BW slots of BW lanes, and a bit with k entries needs
@@ -342,6 +373,7 @@ hipError_t launch_freeze_round(const DevProblem& p, const double* lb, double mar
 // The reference's own float trajectory (anneal_branch): branch b's spins xs[b][bit order]
 // (bytes), residuals rs[b][ray] (FP64) and splitmix64 state sm[b] in global memory; one
 // launch runs sweeps [sweep_begin, sweep_end), the first starting from x = 0.
+hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t entries, hipStream_t st);
 hipError_t launch_ray_ref(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
                           int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
 // The reference's own integer trajectory (wising::anneal), one wave per replica with its

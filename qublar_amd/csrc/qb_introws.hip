@@ -222,7 +222,10 @@ hipError_t launch_int_ref_rows(const DevGraph& g, int R, int waves, bool lds_row
 // of a class reads a field that the class changes, so one barrier per step suffices --
 // while the draw waves make the next step's draws. int_sweep_kernel gives a replica one wave,
 // which decides up to 64 bits, draws for them and walks the flips' rows in L2 one after the
-// other: 0.9 us a class at n = 800, degree 48, 18 classes, where this takes 0.36.
+// other. At n = 800, degree 48, 18 classes and 16 replicas, 1,000 sweeps take 17.2 ms there and
+// 8.4 here (0.95 and 0.47 us a class); what is left is a step's chain of draw, LDS reads and
+// barrier. Draws split over two groups of waves took 9.4 ms, 12 step waves 9.4, 4 step waves
+// 8.8, the next step's bits read ahead 9.2.
 template <bool LDS_ROWS>
 __global__ void __launch_bounds__(kWideBlock) int_wide_kernel(DevGraph g, uint64_t seed_base, const double* beta,
                                                               int sweep_begin, int sweep_end, int init,

@@ -1875,166 +1875,6 @@ hipError_t launch_int_ref(const DevGraph& g, int R, uint64_t seed_base, const do
     return hipGetLastError();
 }
 
-// ---- the reference's own float trajectory (anneal_branch, src/ising_recon.hpp:119-143) ----
-// Branch b anneals from x = 0, r = -d with seed b + 1 + seed_offset: bits in index order,
-// dE = local_field_dE (lin delta, then w (r a + a^2 / 2) per entry with a = a_k delta in CSR
-// order, then lambda (+-1) per neighbour in CSR order), one splitmix64 stream drawn only
-// for uphill proposals, a flip iff dE <= 0 or u < exp(-dE / T), and on a flip r += a_k delta
-// per entry. One wave per branch; x (bytes, bit order) and r (FP64) of a branch live in
-// global memory, read through the CU's L1 (a wave sees its own completed stores). As in the
-// integer trajectory, the wave evaluates the next 64 bits at once -- each lane sums its
-// bit's dE alone, in the reference's order -- and the first accepted bit is the loop's next
-// flip. A flip of a bit with rays ends the window; after a ray-free bit's flip the later
-// lanes only sum their neighbour terms again (the last part of the reference's sum) and
-// decide anew. Draw keys and counters of unions (draw_bit, draw_key) do not apply here.
-__device__ __forceinline__ bool ref_accept_f(uint64_t u53, double dE, double T) {
-    const double x = -dE / T;
-    const double u = double(u53) * 0x1.0p-53;
-    if (!(x > -80.0)) return u < qexp(x);
-    constexpr double kBand = 0x1.0p-14;
-    const double e = double(__builtin_amdgcn_exp2f(float(x) * 1.44269504f));
-    if (u < e * (1.0 - kBand)) return true;
-    if (u > e * (1.0 + kBand)) return false;
-    return u < qexp(x);
-}
-
-// A launch runs sweeps [sweep_begin, sweep_end); the first one starts every branch from
-// x = 0, r = -d and its seed's splitmix64 state, a later one continues from the x, r and
-// state (sm[b]) the previous launch left, so the split never changes the trajectory.
-__global__ void __launch_bounds__(256) ray_ref_kernel(DevProblem p, int R, uint64_t seed_offset, const double* temp,
-                                                       int sweep_begin, int sweep_end, uint8_t* xs, double* rs,
-                                                       uint64_t* sm) {
-    const int w = int(threadIdx.x) / 64, lane = int(threadIdx.x) % 64;
-    const int b = int(blockIdx.x) * 4 + w;
-    if (b >= R) return;   // the whole wave leaves; waves never sync with each other
-    const int n = p.n;
-    uint8_t* x = xs + size_t(b) * size_t(n);
-    double* r = rs + size_t(b) * size_t(p.n_rays);
-    uint64_t st;
-    if (sweep_begin == 0) {
-        for (int i = lane; i < n; i += 64) x[i] = 0;
-        for (int k = lane; k < p.n_rays; k += 64) r[k] = -p.d[k];
-        st = (uint64_t(b) + 1u + seed_offset) * 0x2545F4914F6CDD1Dull + 1;
-    } else {
-        st = sm[b];
-    }
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-    __builtin_amdgcn_wave_barrier();
-    const uint64_t below = (uint64_t(1) << lane) - 1u;
-    for (int sweep = sweep_begin; sweep < sweep_end; ++sweep) {
-        const double T = temp[sweep];
-        int i0 = 0;
-        while (i0 < n) {
-            const int i = i0 + lane;
-            const bool valid = i < n;
-            const int pos = valid ? p.bit_pos[i] : 0;
-            double dE = 0.0, base = 0.0;   // base: the sum up to the neighbour terms
-            const int xi = valid ? int(x[i]) : 0;
-            // each lane's column bounds and update order, kept for the flip
-            const int c0 = valid ? p.col_ptr[pos] : 0, c1 = valid ? p.col_ptr[pos + 1] : 0;
-            const int seq = valid ? int(p.seq_update[pos]) : 0;
-            constexpr int kChunk = 8;
-            if (valid) {
-                // eight entries' loads, then their residuals, in flight together; the sum
-                // itself stays in CSR order
-                const double delta = xi ? -1.0 : 1.0;
-                dE = p.lin[pos] * delta;
-                const int k1 = c1;
-                for (int kb = c0; kb < k1; kb += kChunk) {
-                    RayEnt e[kChunk];
-                    double rv[kChunk];
-#pragma unroll
-                    for (int u = 0; u < kChunk; ++u) e[u] = p.ent[min(kb + u, k1 - 1)];
-#pragma unroll
-                    for (int u = 0; u < kChunk; ++u) rv[u] = r[e[u].ray];
-#pragma unroll
-                    for (int u = 0; u < kChunk; ++u) {
-                        if (kb + u >= k1) break;
-                        const double a = double(e[u].a) * delta;
-                        dE += e[u].w * (rv[u] * a + 0.5 * a * a);
-                    }
-                }
-                base = dE;
-                const int q1 = p.nb_ptr[pos + 1];
-                for (int qb = p.nb_ptr[pos]; qb < q1; qb += kChunk) {
-                    int xv[kChunk];
-#pragma unroll
-                    for (int u = 0; u < kChunk; ++u) xv[u] = x[p.nb_bit[min(qb + u, q1 - 1)]];
-#pragma unroll
-                    for (int u = 0; u < kChunk; ++u) {
-                        if (qb + u >= q1) break;
-                        dE += p.lambda * (xv[u] != xi ? -1.0 : 1.0);
-                    }
-                }
-            }
-            // decisions of the lanes in todo (lanes >= lo) on the current state, the k-th
-            // uphill one drawing st + k gamma
-            uint64_t todo = ~uint64_t(0), m_up = 0, m_acc = 0;
-            auto decide = [&]() {
-                const bool mine = valid && ((todo >> lane) & 1u);
-                const bool up = mine && dE > 0.0;
-                m_up = __ballot(up) & todo;
-                bool acc = mine && dE <= 0.0;
-                if (up) acc = ref_accept_f(mix64(st + uint64_t(__popcll(m_up & below) + 1) * kGamma) >> 11, dE, T);
-                m_acc = __ballot(acc) & todo;
-            };
-            decide();
-            for (;;) {
-                if (m_acc == 0) {
-                    st += uint64_t(__popcll(m_up)) * kGamma;
-                    i0 += 64;
-                    break;
-                }
-                const int js = __builtin_ctzll(m_acc);
-                const uint64_t upto = js == 63 ? ~uint64_t(0) : (uint64_t(2) << js) - 1u;
-                st += uint64_t(__popcll(m_up & upto)) * kGamma;
-                const int fi = i0 + js;
-                const int k0 = __shfl(c0, js), k1 = __shfl(c1, js), seq_f = __shfl(seq, js);
-                const int xf = __shfl(xi, js);
-                const double delta = xf ? -1.0 : 1.0;
-                if (!seq_f) {
-                    for (int k = k0 + lane; k < k1; k += 64) r[p.ent[k].ray] += double(p.ent[k].a) * delta;
-                } else if (lane == 0) {   // a ray repeats in the column: its additions in CSR order
-                    for (int k = k0; k < k1; ++k) r[p.ent[k].ray] += double(p.ent[k].a) * delta;
-                }
-                if (lane == 0) x[fi] = uint8_t(xf ^ 1);
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
-                __builtin_amdgcn_wave_barrier();
-                todo = ~upto;
-                if (k1 > k0 || todo == 0) {   // residuals changed (or the window is done)
-                    i0 = fi + 1;
-                    break;
-                }
-                // A ray-free bit flipped: no residual changed, so a later lane's sum up to its
-                // neighbour terms stands; only those terms are summed again, in order.
-                if (valid && ((todo >> lane) & 1u)) {
-                    dE = base;
-                    const int q1 = p.nb_ptr[pos + 1];
-                    for (int qb = p.nb_ptr[pos]; qb < q1; qb += kChunk) {
-                        int xv[kChunk];
-#pragma unroll
-                        for (int u = 0; u < kChunk; ++u) xv[u] = x[p.nb_bit[min(qb + u, q1 - 1)]];
-#pragma unroll
-                        for (int u = 0; u < kChunk; ++u) {
-                            if (qb + u >= q1) break;
-                            dE += p.lambda * (xv[u] != xi ? -1.0 : 1.0);
-                        }
-                    }
-                }
-                decide();
-            }
-        }
-    }
-    if (lane == 0) sm[b] = st;
-}
-
-hipError_t launch_ray_ref(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
-                          int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st) {
-    ray_ref_kernel<<<unsigned((R + 3) / 4), 256, 0, st>>>(p, R, seed_offset, temp, sweep_begin, sweep_end, xs, rs,
-                                                          sm);
-    return hipGetLastError();
-}
-
 // ---- the team barrier's visibility, checked on the device ---------------------------------
 // The sweep relies on a team's plain stores, drained before its barrier, being seen by the
 // L2-hitting loads of every member after it. This kernel exercises exactly that: each

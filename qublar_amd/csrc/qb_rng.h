@@ -190,15 +190,18 @@ __device__ __forceinline__ uint64_t mix64(uint64_t z) {
 // most an ulp or two, so a decision can differ from the host's only for a u within that
 // distance of the exponential.
 template <typename I>
-__device__ __forceinline__ bool ref_accept(uint64_t u53, I dE, double T, double nrT) {
+__device__ __forceinline__ bool ref_accept_u(double u, I dE, double T, double nrT) {
     const double xa = double(dE) * nrT;
-    const double u = double(u53) * 0x1.0p-53;
     if (!(xa > -79.0)) return u < qexp(-double(dE) / T);   // only u = 0 can pass below e^-79
     constexpr double kBand = 0x1.0p-14;
     const double e = double(__builtin_amdgcn_exp2f(float(xa) * 1.44269504f));
     if (u < e * (1.0 - kBand)) return true;
     if (u > e * (1.0 + kBand)) return false;
     return u < qexp(-double(dE) / T);
+}
+template <typename I>
+__device__ __forceinline__ bool ref_accept(uint64_t u53, I dE, double T, double nrT) {
+    return ref_accept_u(double(u53) * 0x1.0p-53, dE, T, nrT);
 }
 #endif
 
