@@ -434,21 +434,19 @@ struct DevQuboBatch {
     const int32_t* inst_pos;     // n_instances + 1
     const int32_t* inst_cls;     // n_instances + 1 offsets into cls_ptr
     const int32_t* cls_ptr;      // per instance: its n_classes + 1 class bounds (global positions)
-    const int32_t* row_ptr;      // total bits + 1
-    const int32_t* col;          // neighbour position
-    const float* J;              // coupling per entry
     const float* h;              // field per position
     const int32_t* bit_id;       // per position: the bit's index inside its instance (draw counter)
     const uint64_t* seed;        // per instance
-    // The rows again, sliced by 64 positions of a class (a wave's bits in one pass) and
+    // The rows, sliced by 64 positions of a class (a wave's bits in one pass) and
     // stored entry-major: entry u of tile t's lane l at tile_ptr[t] + 64 u + l, so one load
     // of a wave reads 64 consecutive words. Tile t of class c is class_tile[c] + (pos - lo) / 64.
     const int32_t* class_tile;   // per class (global class index)
-    const int32_t* tile_ptr;     // per tile
-    const int32_t* tcol;         // neighbour position
-    const float* tJ;             // coupling
+    const int32_t* tile_ptr;     // per tile, and the end of the last
+    const int32_t* tile_pos;     // its first position, and the batch's bits behind the last
+    const int32_t* tcol;         // neighbour position in the instance (the bit itself past a row's end)
+    const float* tJ;             // coupling (0 past a row's end)
 };
-constexpr int kQuboBlock = 256;      // threads of the energy kernel
+constexpr int kQuboEnergyBlock = 1024;   // threads of the energy kernel
 constexpr int kQuboLdsBytes = 65536;  // LDS spin words of one annealing job
 // block: 256 or 1024 threads per workgroup (one bit per thread in a class pass).
 // The persistent kernel's job queues, one per XCD: jobs [begin[x], begin[x + 1]) of
@@ -462,7 +460,8 @@ struct QuboQueues {
 hipError_t launch_qubo_batch(const DevQuboBatch& q, int rb, int block, uint32_t* masks, const double* beta,
                              int n_sweeps, unsigned* queue, const QuboQueues& segs, int workgroups, hipStream_t st);
 int qubo_blocks_per_cu(int rb, int block);
-hipError_t launch_qubo_energy(const DevQuboBatch& q, const uint32_t* masks, double* energy, hipStream_t st);
+// The energies of every job's replicas, at most rb of them to a job.
+hipError_t launch_qubo_energy(const DevQuboBatch& q, int rb, const uint32_t* masks, double* energy, hipStream_t st);
 // p[0 .. n) = v: a kernel, so a recorded graph holds no memset node.
 hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t st);
 

@@ -11,9 +11,8 @@
 // order, a class is a set of independent flips, and the workgroup syncs between classes.
 //
 // Inside a class each lane takes one bit for all the job's replicas: it walks the bit's
-// CSR row once, kRowChunk neighbours at a time (columns and couplings, then the
-// neighbours' spin words, all in flight together), and adds each coupling into the
-// accumulator of every replica whose neighbour spin is set -- in row order, per replica.
+// row once (walk_row) and adds each coupling into the accumulator of every replica whose
+// neighbour spin is set -- in row order, per replica.
 // The spin words of a job (bit r of word i = replica r0 + r's x_i) live in the
 // workgroup's LDS while it anneals (global memory only for instances too large for it),
 // so the random reads of neighbours' spins never leave the CU.
@@ -28,8 +27,6 @@
 #include "qb_rng.h"
 
 namespace qb {
-
-constexpr int kRowChunk = 16;
 
 // Spin words of a job in LDS: one byte per bit up to 8 replicas per job, 16 or 32 bits
 // beyond; kQuboLdsBytes of them hold instances up to kQuboLdsBytes / sizeof(word) bits.
@@ -50,6 +47,58 @@ struct LdsWord<16> {
     using type = uint16_t;
 };
 
+// Bits a spin word is shifted up by: four replicas to a byte lie in its upper half, where
+// walk_row wants them.
+template <int RB, typename W>
+constexpr int word_shift() {
+    return RB == 4 && sizeof(W) == 1 ? 4 : 0;
+}
+
+// N entries of a tile's rows: columns and couplings, then the neighbours' spin words, all in
+// flight together; each coupling goes into the accumulator of every replica whose neighbour
+// spin is set, in row order, as fma(w, x_j, acc): w x_j is exact, so each addition rounds once
+// as acc + w does, and an unset neighbour -- or a padding entry, whose coupling is zero --
+// leaves acc (up to the sign of an exact zero, which no decision sees).
+//
+// The sums bound the sweep, instruction by instruction. With four replicas to a byte, a
+// multiplication spreads the nibble to one bit a byte and each replica's x_j, as 0 or 2.0, is
+// one byte moved to the top of a double: two instructions per (entry, replica) where bit
+// field, conversion and FMA are three (the accumulators hold twice the sums). Rows padded to
+// their tile's longest need no test per entry, and a tile's steps are its own length (16, then
+// 8, 4, 2 and 1 entries), not whole steps of 16. 48 instances of 1,000 to 16,384 bits, degrees
+// 3 to 64, 8 to 32 replicas, 400 sweeps: 86.5 -> 53.7 ms. (x_j as any one exponent bit of a
+// double would save the moved byte too, but factors of 2^-511 and below slow the FMAs: 280.)
+template <int RB, int N, int SHIFT, typename W>
+__device__ __forceinline__ void walk_row(const int* tcol, const float* tJ, const W* mk, double (&acc)[RB]) {
+    const unsigned lane = threadIdx.x % 64;
+    int cj[N];
+    float wj[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        cj[u] = tcol[lane + 64u * u];
+        wj[u] = tJ[lane + 64u * u];
+    }
+    uint32_t mj[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) mj[u] = uint32_t(mk[cj[u]]);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+        const double w = double(wj[u]);
+        if constexpr (SHIFT != 0) {
+            static_assert(RB == 4 && SHIFT == 4);
+            const uint32_t word = (mj[u] * 0x810204u) & 0x40404040u;   // bit 4 + r to bit 8 r + 6
+#pragma unroll
+            for (int r = 0; r < RB; ++r) {
+                const uint32_t hi = __builtin_amdgcn_perm(word, word, (uint32_t(r) << 24) | 0x0C0C0Cu);
+                acc[r] = fma(w, __hiloint2double(int(hi), 0), acc[r]);
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < RB; ++r) acc[r] = fma(w, double((mj[u] >> r) & 1u), acc[r]);
+        }
+    }
+}
+
 // One job's sweeps with its spin words at `mk` (LDS or global), local position index.
 template <int RB, int BLOCK, typename W>
 __device__ __forceinline__ void qubo_job(const DevQuboBatch& q, const QuboJob& jb, W* mk, const double* beta,
@@ -59,41 +108,38 @@ __device__ __forceinline__ void qubo_job(const DevQuboBatch& q, const QuboJob& j
     const int c0 = q.inst_cls[k], c1 = q.inst_cls[k + 1];
     const uint64_t key = q.seed[k];
     const uint32_t pair0 = uint32_t(jb.replica0) / 2u;   // replica0 is a multiple of RB
+    constexpr int kShift = word_shift<RB, W>();
+    constexpr double kUnit = kShift ? 2.0 : 1.0;
     for (int sweep = 0; sweep < n_sweeps; ++sweep) {
         const double b = beta[sweep];
         for (int c = c0; c + 1 < c1; ++c) {
             const int lo = q.cls_ptr[c], hi = q.cls_ptr[c + 1];
             for (int pos = lo + int(threadIdx.x); pos < hi; pos += BLOCK) {
-                const uint32_t mi = mk[pos - bit0];
-                const double hp = double(q.h[pos]);
+                const uint32_t mi = uint32_t(mk[pos - bit0]) >> kShift;
+                const double hp = double(q.h[pos]) * kUnit;
                 double acc[RB];
 #pragma unroll
                 for (int r = 0; r < RB; ++r) acc[r] = hp;
-                const int deg = q.row_ptr[pos + 1] - q.row_ptr[pos];
-                const int* tc = q.tcol + q.tile_ptr[q.class_tile[c] + (pos - lo) / 64] + ((pos - lo) & 63);
-                const float* tw = q.tJ + (tc - q.tcol);
-                for (int ea = 0; ea < deg; ea += kRowChunk) {
-                    int cj[kRowChunk];
-                    float wj[kRowChunk];
+                const int tile = q.class_tile[c] + __builtin_amdgcn_readfirstlane((pos - lo) >> 6);
+                const int at = q.tile_ptr[tile], end = q.tile_ptr[tile + 1];
+                int e = at;
+                for (; end - e >= 64 * 16; e += 64 * 16) walk_row<RB, 16, kShift>(q.tcol + e, q.tJ + e, mk, acc);
+                if (end - e >= 64 * 8) {
+                    walk_row<RB, 8, kShift>(q.tcol + e, q.tJ + e, mk, acc);
+                    e += 64 * 8;
+                }
+                if (end - e >= 64 * 4) {
+                    walk_row<RB, 4, kShift>(q.tcol + e, q.tJ + e, mk, acc);
+                    e += 64 * 4;
+                }
+                if (end - e >= 64 * 2) {
+                    walk_row<RB, 2, kShift>(q.tcol + e, q.tJ + e, mk, acc);
+                    e += 64 * 2;
+                }
+                if (end - e >= 64) walk_row<RB, 1, kShift>(q.tcol + e, q.tJ + e, mk, acc);
+                if constexpr (kShift != 0) {
 #pragma unroll
-                    for (int u = 0; u < kRowChunk; ++u) {
-                        const int e = min(ea + u, deg - 1);
-                        cj[u] = tc[64 * e];
-                        wj[u] = tw[64 * e];
-                    }
-                    uint32_t mj[kRowChunk];
-#pragma unroll
-                    for (int u = 0; u < kRowChunk; ++u) mj[u] = ea + u < deg ? uint32_t(mk[cj[u] - bit0]) : 0u;
-                    // acc += w where the neighbour's spin is set, as fma(w, x_j, acc): w * 1 and
-                    // w * 0 are exact, so each addition rounds once as acc + w does, and an
-                    // unset neighbour leaves acc (up to the sign of an exact zero, which no
-                    // decision sees) -- three instructions per (entry, replica), no select
-#pragma unroll
-                    for (int u = 0; u < kRowChunk; ++u) {
-                        const double w = double(wj[u]);
-#pragma unroll
-                        for (int r = 0; r < RB; ++r) acc[r] = fma(w, double((mj[u] >> r) & 1u), acc[r]);
-                    }
+                    for (int r = 0; r < RB; ++r) acc[r] *= 1.0 / kUnit;
                 }
                 const uint32_t bit = uint32_t(q.bit_id[pos]);
                 uint32_t flips = 0;
@@ -109,7 +155,7 @@ __device__ __forceinline__ void qubo_job(const DevQuboBatch& q, const QuboJob& j
                         }
                     }
                 }
-                if (flips) mk[pos - bit0] = W(mi ^ flips);
+                if (flips) mk[pos - bit0] = W((mi ^ flips) << kShift);
             }
             __syncthreads();
         }
@@ -153,7 +199,7 @@ __global__ void __launch_bounds__(BLOCK) qubo_batch_kernel(DevQuboBatch q, uint3
             for (int i = int(threadIdx.x); i < n; i += BLOCK) lmask[i] = W(0);
             __syncthreads();
             qubo_job<RB, BLOCK, W>(q, jb, lmask, beta, n_sweeps);
-            for (int i = int(threadIdx.x); i < n; i += BLOCK) gm[i] = uint32_t(lmask[i]);
+            for (int i = int(threadIdx.x); i < n; i += BLOCK) gm[i] = uint32_t(lmask[i]) >> word_shift<RB, W>();
             __syncthreads();
         } else {
             qubo_job<RB, BLOCK, uint32_t>(q, jb, gm, beta, n_sweeps);
@@ -161,34 +207,66 @@ __global__ void __launch_bounds__(BLOCK) qubo_batch_kernel(DevQuboBatch q, uint3
     }
 }
 
-// FP64 energy of every replica of every job: one workgroup per job, thread t sums
-// positions t, t + kQuboBlock, ... for each of the job's replicas, then a tree
-// reduction per replica.
-__global__ void __launch_bounds__(kQuboBlock) qubo_energy_kernel(DevQuboBatch q, const uint32_t* masks,
-                                                                 double* energy) {
-    __shared__ double part[kQuboBlock];
+// FP64 energy of the replicas of every job, four of them per workgroup: a wave takes every
+// 16th tile of the instance, a lane a bit of it for the four replicas, so a row is read once
+// for all of them in whole lines, eight entries in flight; then a tree over the lanes and the
+// waves. Bound by the latency of the spin words' gathers. 48 instances of 1,000 to 16,384
+// bits, 8 to 32 replicas: 0.24 ms, where a workgroup per job that walked its replicas one
+// after the other, a row per lane, took 5.6.
+__global__ void __launch_bounds__(kQuboEnergyBlock) qubo_energy_kernel(DevQuboBatch q, const uint32_t* masks,
+                                                                       double* energy) {
+    constexpr int kR = 4, kFlight = 8, kWaves = kQuboEnergyBlock / 64;
+    __shared__ double part[kR][kWaves];
     const QuboJob jb = q.jobs[blockIdx.x];
-    const int k = jb.instance;
+    const int r0 = int(blockIdx.y) * kR;
+    if (r0 >= jb.replicas) return;   // the whole workgroup leaves
+    const int k = jb.instance, lane = int(threadIdx.x) % 64;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / 64);
     const uint32_t* mk = masks + jb.mask_offset;
-    const int bit0 = q.inst_pos[k], bit1 = q.inst_pos[k + 1];
-    for (int r = 0; r < jb.replicas; ++r) {
-        double e = 0.0;
-        for (int pos = bit0 + int(threadIdx.x); pos < bit1; pos += kQuboBlock) {
-            if (!((mk[pos - bit0] >> r) & 1u)) continue;
-            double f = double(q.h[pos]);
-            double pair = 0.0;
-            for (int i = q.row_ptr[pos]; i < q.row_ptr[pos + 1]; ++i)
-                if ((mk[q.col[i] - bit0] >> r) & 1u) pair += double(q.J[i]);
-            e += f + 0.5 * pair;
+    const int bit0 = q.inst_pos[k];
+    const int t1 = q.class_tile[q.inst_cls[k + 1] - 1];
+    double e[kR] = {};
+    for (int t = q.class_tile[q.inst_cls[k]] + wave; t < t1; t += kWaves) {
+        const int pos = q.tile_pos[t] + lane;
+        const bool valid = pos < q.tile_pos[t + 1];
+        const uint32_t mi = valid ? mk[pos - bit0] >> r0 : 0u;
+        double pair[kR] = {};
+        const int at = q.tile_ptr[t], end = q.tile_ptr[t + 1];
+        for (int i = at; i < end; i += 64 * kFlight) {
+            int cj[kFlight];
+            float wj[kFlight];
+            uint32_t mj[kFlight];
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) {
+                const int from = min(i + 64 * u, end - 64) + lane;
+                cj[u] = q.tcol[from];
+                wj[u] = q.tJ[from];
+            }
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u) mj[u] = i + 64 * u < end ? mk[cj[u]] >> r0 : 0u;
+#pragma unroll
+            for (int u = 0; u < kFlight; ++u)
+#pragma unroll
+                for (int r = 0; r < kR; ++r) pair[r] = fma(double(wj[u]), double((mj[u] >> r) & 1u), pair[r]);
         }
-        part[threadIdx.x] = e;
-        __syncthreads();
-        for (int w = kQuboBlock / 2; w > 0; w /= 2) {
-            if (int(threadIdx.x) < w) part[threadIdx.x] += part[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) energy[jb.energy_offset + r] = part[0];
-        __syncthreads();
+        const double h = valid ? double(q.h[pos]) : 0.0;
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+            if ((mi >> r) & 1u) e[r] += h + 0.5 * pair[r];
+    }
+#pragma unroll
+    for (int r = 0; r < kR; ++r) {
+#pragma unroll
+        for (int d = 32; d > 0; d /= 2) e[r] += __shfl_down(e[r], unsigned(d));
+        if (lane == 0) part[r][wave] = e[r];
+    }
+    __syncthreads();
+    const int r = int(threadIdx.x) / kWaves, w = int(threadIdx.x) % kWaves;   // 16 lanes a replica
+    if (int(threadIdx.x) < kR * kWaves) {
+        double v = part[r][w];
+#pragma unroll
+        for (int d = kWaves / 2; d > 0; d /= 2) v += __shfl_down(v, unsigned(d), kWaves);
+        if (w == 0 && r0 + r < jb.replicas) energy[jb.energy_offset + r0 + r] = v;
     }
 }
 
@@ -240,8 +318,8 @@ hipError_t launch_fill_u32(uint32_t* p, size_t n, uint32_t v, hipStream_t st) {
     return hipGetLastError();
 }
 
-hipError_t launch_qubo_energy(const DevQuboBatch& q, const uint32_t* masks, double* energy, hipStream_t st) {
-    qubo_energy_kernel<<<q.n_jobs, kQuboBlock, 0, st>>>(q, masks, energy);
+hipError_t launch_qubo_energy(const DevQuboBatch& q, int rb, const uint32_t* masks, double* energy, hipStream_t st) {
+    qubo_energy_kernel<<<dim3(unsigned(q.n_jobs), unsigned((rb + 3) / 4)), kQuboEnergyBlock, 0, st>>>(q, masks, energy);
     return hipGetLastError();
 }
 
