@@ -2081,6 +2081,7 @@ struct qb_qubo_batch {
     std::vector<int32_t> e_off;       // per instance: offset of its replicas in the energy output
     std::vector<uint64_t> seed;
     int total_replicas = 0;
+    int cus = 0;   // compute units of its device
     DevBuf b_inst_pos, b_inst_cls, b_cls, b_h, b_bit, b_seed, b_ctile, b_tptr, b_tpos, b_tcol, b_tJ;
     struct Jobs {
         DevBuf by_xcd, by_inst;       // the same jobs, grouped by XCD queue and in instance order
@@ -2088,6 +2089,7 @@ struct qb_qubo_batch {
         std::vector<QuboJob> host;    // instance order
         std::vector<int32_t> first;   // per instance: its first job in instance order
         int64_t mask_words = 0;
+        int blocks = 0;   // replica blocks; long ones are two jobs
     };
     std::map<int, std::unique_ptr<Jobs>> jobs;   // by replica block
     DevBuf w_mask, w_beta, w_queue, w_energy;
@@ -2255,6 +2257,9 @@ extern "C" int qb_qubo_batch_create(const qb_qubo_batch_desc* d, qb_qubo_batch**
         hoff += n;
     }
     B->n_total = B->inst_pos.back();
+    hipDeviceProp_t prop;
+    if (int prc = device_props(prop)) return prc;
+    B->cus = prop.multiProcessorCount;
     // the rows sliced by 64 positions of each class, entry-major (padding: the bit itself, J = 0)
     std::vector<int32_t> ctile, tptr, tpos, tcol;
     std::vector<float> tJ;
@@ -2312,8 +2317,44 @@ extern "C" int qb_qubo_batch_destroy(qb_qubo_batch* b) {
     return QB_OK;
 }
 
-// Jobs at replica block rb: instance k's replicas in blocks of rb, each block a job with
-// its own spin words. Uploaded in instance order, and grouped by XCD queue: instances in
+// The instructions of one sweep of a job, roughly: per bit its draws and decisions, per entry
+// the walk's fixed part and two instructions a replica (four replicas: 350 and 12).
+static int64_t qubo_job_cost(const qb_qubo_batch* B, int k, int replicas) {
+    return int64_t(B->n_bits[size_t(k)]) * (150 + 50 * replicas) + B->entries[size_t(k)] * (4 + 2 * replicas);
+}
+
+// Replicas per job of every instance at replica block rb. A job is one workgroup's from
+// start to end, so a batch of uneven instances lasts as long as its longest job: blocks of four
+// are halved, the longest first, while a whole one takes longer than an even share of the
+// batch on every CU and than the longest half. 48 instances of 1,000 to 16,384 bits, whose
+// longest block of four is 3.8 even shares: 53.7 -> 42.2 ms.
+static std::vector<int> qubo_job_sizes(const qb_qubo_batch* B, int rb) {
+    std::vector<int> size(static_cast<size_t>(B->n_inst), rb);
+    if (rb != 4) return size;
+    std::vector<int> order(static_cast<size_t>(B->n_inst));
+    int64_t total = 0, words = 0;
+    for (int k = 0; k < B->n_inst; ++k) {
+        const int64_t blocks = (B->replicas[size_t(k)] + 3) / 4;
+        order[size_t(k)] = k;
+        total += blocks * qubo_job_cost(B, k, 4);
+        words += blocks * B->n_bits[size_t(k)];
+    }
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int a, int b) { return qubo_job_cost(B, a, 4) > qubo_job_cost(B, b, 4); });
+    const int64_t half = qubo_job_cost(B, order.front(), 2);
+    for (int k : order) {
+        const int64_t whole = qubo_job_cost(B, k, 4);
+        const int64_t blocks = (B->replicas[size_t(k)] + 3) / 4, halves = (B->replicas[size_t(k)] + 1) / 2;
+        words += (halves - blocks) * B->n_bits[size_t(k)];
+        if (whole <= half || whole <= total / std::max(B->cus, 1) || words > INT32_MAX) break;
+        total += halves * qubo_job_cost(B, k, 2) - blocks * whole;
+        size[size_t(k)] = 2;
+    }
+    return size;
+}
+
+// Jobs at replica block rb: instance k's replicas in blocks of rb (or, of a long instance,
+// half of that), each block a job with its own spin words. Uploaded in instance order, and grouped by XCD queue: instances in
 // decreasing cost (rows + entries, times replicas) each go to the least loaded of the
 // eight queues, and a queue lists its instances in that order with each instance's jobs
 // side by side.
@@ -2324,14 +2365,16 @@ static int qubo_jobs_for(qb_qubo_batch* B, int rb, const qb_qubo_batch::Jobs** o
         return QB_OK;
     }
     auto Jb = std::make_unique<qb_qubo_batch::Jobs>();
+    const std::vector<int> size = qubo_job_sizes(B, rb);
     int64_t words = 0;
     for (int k = 0; k < B->n_inst; ++k) {
         Jb->first.push_back(int32_t(Jb->host.size()));
-        for (int r0 = 0; r0 < B->replicas[size_t(k)]; r0 += rb) {
+        Jb->blocks += (B->replicas[size_t(k)] + rb - 1) / rb;
+        for (int r0 = 0; r0 < B->replicas[size_t(k)]; r0 += size[size_t(k)]) {
             QuboJob j{};
             j.instance = k;
             j.replica0 = r0;
-            j.replicas = std::min(rb, B->replicas[size_t(k)] - r0);
+            j.replicas = std::min(size[size_t(k)], B->replicas[size_t(k)] - r0);
             j.mask_offset = int32_t(words);
             j.energy_offset = B->e_off[size_t(k)] + r0;
             words += B->n_bits[size_t(k)];
@@ -2354,6 +2397,11 @@ static int qubo_jobs_for(qb_qubo_batch* B, int rb, const qb_qubo_batch::Jobs** o
         queue_inst[size_t(x)].push_back(k);
         load[size_t(x)] += cost(k);
     }
+    // a queue's longest jobs first, so that none of them starts when the others are done
+    for (auto& inst : queue_inst)
+        std::stable_sort(inst.begin(), inst.end(), [&](int a, int b) {
+            return qubo_job_cost(B, a, size[size_t(a)]) > qubo_job_cost(B, b, size[size_t(b)]);
+        });
     std::vector<QuboJob> by_xcd;
     by_xcd.reserve(Jb->host.size());
     for (int x = 0; x < kXcds; ++x) {
@@ -2565,7 +2613,7 @@ extern "C" int qb_qubo_batch_anneal(qb_qubo_batch* B, const qb_schedule* s, cons
         rep->launches = launches;
         rep->replica_block = rb;
         rep->block = block;
-        rep->jobs = int(Jb->host.size());
+        rep->jobs = Jb->blocks;
         rep->graph_replayed = replayed ? 1 : 0;
         double upd = 0.0;
         for (int k = 0; k < B->n_inst; ++k) upd += double(B->replicas[size_t(k)]) * double(B->n_bits[size_t(k)]);

@@ -51,7 +51,7 @@ struct LdsWord<16> {
 // walk_row wants them.
 template <int RB, typename W>
 constexpr int word_shift() {
-    return RB == 4 && sizeof(W) == 1 ? 4 : 0;
+    return RB <= 4 && sizeof(W) == 1 ? 4 : 0;
 }
 
 // N entries of a tile's rows: columns and couplings, then the neighbours' spin words, all in
@@ -85,7 +85,7 @@ __device__ __forceinline__ void walk_row(const int* tcol, const float* tJ, const
     for (int u = 0; u < N; ++u) {
         const double w = double(wj[u]);
         if constexpr (SHIFT != 0) {
-            static_assert(RB == 4 && SHIFT == 4);
+            static_assert(RB <= 4 && SHIFT == 4);
             const uint32_t word = (mj[u] * 0x810204u) & 0x40404040u;   // bit 4 + r to bit 8 r + 6
 #pragma unroll
             for (int r = 0; r < RB; ++r) {
@@ -198,7 +198,8 @@ __global__ void __launch_bounds__(BLOCK) qubo_batch_kernel(DevQuboBatch q, uint3
             // the job's spins live in LDS from all-zero x; written out once at the end
             for (int i = int(threadIdx.x); i < n; i += BLOCK) lmask[i] = W(0);
             __syncthreads();
-            qubo_job<RB, BLOCK, W>(q, jb, lmask, beta, n_sweeps);
+            if (RB == 4 && jb.replicas <= 2) qubo_job<2, BLOCK, W>(q, jb, lmask, beta, n_sweeps);
+            else qubo_job<RB, BLOCK, W>(q, jb, lmask, beta, n_sweeps);
             for (int i = int(threadIdx.x); i < n; i += BLOCK) gm[i] = uint32_t(lmask[i]) >> word_shift<RB, W>();
             __syncthreads();
         } else {
