@@ -28,34 +28,84 @@ constexpr int kDenseWin = 64;
 constexpr int kRankChunk = 8;
 constexpr int kFieldGroup = 4;   // fields a thread updates together (i, i + block, ...)
 
-// Fields i = g0 + q STRIDE (q < kFieldGroup, i < n) from scratch:
-// h_i + sum_j x_j Q_ji in FP64, j ascending (Q_ji = Q_ij), additions of unset bits
-// skipped; every field's loads of a 16-column chunk in flight together.
-template <int STRIDE = kDenseBlock>
-__device__ __forceinline__ void scratch_fields(const DevDense& d, const uint8_t* x, int g0, double (&s)[kFieldGroup]) {
-    constexpr int kChunk = 16;
-    const int n = d.n;
-    int col[kFieldGroup];
-#pragma unroll
-    for (int q = 0; q < kFieldGroup; ++q) {
-        col[q] = min(g0 + q * STRIDE, n - 1);
-        s[q] = double(d.h[col[q]]);
+constexpr int kListBits = 2 * kDenseWin * kDenseWin;   // 16-bit entries in one staging buffer
+
+// The list of the set bits j of x in [p0, p0 + kListBits), less p0, in order; their number.
+__device__ __forceinline__ int list_set_bits(const uint8_t* x, int n, int p0, uint16_t* list, int* s_count) {
+    __syncthreads();   // the list's last readers are done
+    if (threadIdx.x < 64) {
+        const int lane = int(threadIdx.x);
+        int count = 0;
+        for (int j0 = p0; j0 < min(n, p0 + kListBits); j0 += 64) {
+            const bool set = j0 + lane < n && x[min(j0 + lane, n - 1)];
+            const uint64_t m = __ballot(set);
+            if (set) list[count + __popcll(m & ((uint64_t(1) << lane) - 1u))] = uint16_t(j0 + lane - p0);
+            count += __popcll(m);
+        }
+        if (lane == 0) *s_count = count;
     }
-    for (int j0 = 0; j0 < n; j0 += kChunk) {
-        float v[kFieldGroup][kChunk];
+    __syncthreads();
+    return *s_count;
+}
+
+// s plus the listed rows' elements at column col, in the list's order, ROWS rows' loads in
+// flight while the ROWS before them are added.
+template <int ROWS>
+__device__ __forceinline__ double add_listed(const DevDense& d, const float* Qp, const uint16_t* list, int count,
+                                             int col, double s) {
+    const int lane = int(threadIdx.x) % 64;
+    float va[ROWS], vb[ROWS];
+    auto load = [&](float (&v)[ROWS], int c) {
+        const int mine = list[min(c + lane, count - 1)];   // past the last row: read again, not added
 #pragma unroll
-        for (int u = 0; u < kChunk; ++u)
+        for (int u = 0; u < ROWS; ++u)
+            v[u] = (Qp + size_t(__builtin_amdgcn_readlane(mine, u)) * size_t(d.n))[unsigned(col)];
+    };
+    auto add = [&](const float (&v)[ROWS], int c) {
+        if (c + ROWS <= count) {
 #pragma unroll
-            for (int q = 0; q < kFieldGroup; ++q) v[q][u] = d.Q[size_t(min(j0 + u, n - 1)) * size_t(n) + size_t(col[q])];
+            for (int u = 0; u < ROWS; ++u) s += double(v[u]);
+        } else {
 #pragma unroll
-        for (int u = 0; u < kChunk; ++u) {
-            const bool set = j0 + u < n && x[min(j0 + u, n - 1)];
-#pragma unroll
-            for (int q = 0; q < kFieldGroup; ++q) {
-                const double nxt = s[q] + double(v[q][u]);
-                s[q] = set ? nxt : s[q];
+            for (int u = 0; u < ROWS; ++u) {
+                const double next = s + double(v[u]);
+                s = c + u < count ? next : s;
             }
         }
+    };
+    load(va, 0);
+    for (int c = 0; c < count; c += 2 * ROWS) {
+        load(vb, c + ROWS);
+        add(va, c);
+        load(va, c + 2 * ROWS);
+        add(vb, c + ROWS);
+    }
+    return s;
+}
+
+// put(i, h_i + sum_j x_j Q_ji) for the fields i in [first, last), in FP64, j ascending (Q_ji =
+// Q_ij): a thread a field, the set bits' rows alone, from a list in `list` (one staging
+// buffer). Called by every thread of the workgroup. Bound by the rows' bytes and latency, so
+// as many loads are in flight as registers hold (32 twice, and 16 twice where 1,024 threads
+// leave 128 registers). 2,048 bits, 4 workgroups a replica, 32 replicas: 49 us, where the loads
+// of every row, set or not, 16 for four columns each, took 277.
+template <int THREADS, typename F>
+__device__ __forceinline__ void scratch_fields(const DevDense& d, const uint8_t* x, uint16_t* list, int first,
+                                               int last, F&& put) {
+    __shared__ int s_count;
+    int listed = -1, count = 0;
+    for (int g = first; g < last; g += THREADS) {
+        const int i = g + int(threadIdx.x), col = min(i, last - 1);
+        const bool wave_live = g + int(threadIdx.x & ~63u) < last;
+        double s = double(d.h[col]);
+        for (int p0 = 0; p0 < d.n; p0 += kListBits) {
+            if (listed != p0) {
+                count = __builtin_amdgcn_readfirstlane(list_set_bits(x, d.n, p0, list, &s_count));
+                listed = p0;
+            }
+            if (wave_live && count > 0) s = add_listed<THREADS <= 512 ? 32 : 16>(d, d.Q + size_t(p0) * size_t(d.n), list, count, col, s);
+        }
+        if (i < last) put(i, s);
     }
 }
 
@@ -216,31 +266,20 @@ __global__ void __launch_bounds__(kDenseBlock) dense_anneal_kernel(DevDense d, c
             nbuf ^= 1;
         }
         if (recompute_every > 0 && (sweep + 1) % recompute_every == 0) {
-            // f = h + Q x from scratch in FP64, j ascending (column i of Q = row i)
-            for (int g0 = tid; g0 < n; g0 += kFieldGroup * kDenseBlock) {
-                double sc[kFieldGroup];
-                scratch_fields(d, x, g0, sc);   // reads x and Q only, so fields may change meanwhile
-#pragma unroll
-                for (int q = 0; q < kFieldGroup; ++q)
-                    if (g0 + q * kDenseBlock < n) f[g0 + q * kDenseBlock] = T(sc[q]);
-            }
+            // f = h + Q x from scratch in FP64, j ascending (column i of Q = row i); it reads x and
+            // Q only, so fields may change meanwhile. The next window is staged in buffer nbuf.
+            scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk + (nbuf ^ 1) * kDenseWin * kDenseWin), 0,
+                                        n, [&](int i, double v) { f[i] = T(v); });
             __syncthreads();
         }
     }
     // outputs: spins, the FP64 energy and max |f_carried - f_scratch|
     double e = 0.0, err = 0.0;
-    for (int g0 = tid; g0 < n; g0 += kFieldGroup * kDenseBlock) {
-        double sc[kFieldGroup];
-        scratch_fields(d, x, g0, sc);
-#pragma unroll
-        for (int q = 0; q < kFieldGroup; ++q) {
-            const int i = g0 + q * kDenseBlock;
-            if (i >= n) continue;
-            err = fmax(err, fabs(double(f[i]) - sc[q]));
-            if (x[i]) e += double(d.h[i]) + 0.5 * (sc[q] - double(d.h[i]));
-            x_out[size_t(blockIdx.x) * size_t(n) + size_t(i)] = x[i];
-        }
-    }
+    scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk), 0, n, [&](int i, double v) {
+        err = fmax(err, fabs(double(f[i]) - v));
+        if (x[i]) e += double(d.h[i]) + 0.5 * (v - double(d.h[i]));
+        x_out[size_t(blockIdx.x) * size_t(n) + size_t(i)] = x[i];
+    });
     for (int o = 32; o > 0; o /= 2) {
         e += __shfl_down(e, o);
         err = fmax(err, __shfl_down(err, o));
@@ -637,14 +676,11 @@ __global__ void __launch_bounds__(kDenseTeamBlock) dense_team_kernel(DevDense d,
         }
         if (recompute_every > 0 && (sweep + 1) % recompute_every == 0) {
             // every wave is past the sweep's last window: the fields from scratch in FP64
+            // (the next two windows are staged in the two buffers other than the last window's)
             __syncthreads();
-            for (int g0 = ib + tid; g0 < ie; g0 += kFieldGroup * kDenseTeamBlock) {
-                double sc[kFieldGroup];
-                scratch_fields<kDenseTeamBlock>(d, x, g0, sc);
-#pragma unroll
-                for (int qq = 0; qq < kFieldGroup; ++qq)
-                    if (g0 + qq * kDenseTeamBlock < ie) f[g0 + qq * kDenseTeamBlock - ib] = T(sc[qq]);
-            }
+            const int last_buf = ((sweep + 1) * n_win - 1) % 3;
+            scratch_fields<kDenseTeamBlock>(d, x, reinterpret_cast<uint16_t*>(blk + last_buf * kDenseWin * kDenseWin),
+                                            ib, ie, [&](int i, double v) { f[i - ib] = T(v); });
             __syncthreads();
         }
     }
@@ -652,18 +688,11 @@ __global__ void __launch_bounds__(kDenseTeamBlock) dense_team_kernel(DevDense d,
     if (s_abort) return;
     // outputs: this part's spins, its share of the FP64 energy and of max |f - f_scratch|
     double e = 0.0, er = 0.0;
-    for (int g0 = ib + tid; g0 < ie; g0 += kFieldGroup * kDenseTeamBlock) {
-        double sc[kFieldGroup];
-        scratch_fields<kDenseTeamBlock>(d, x, g0, sc);
-#pragma unroll
-        for (int q = 0; q < kFieldGroup; ++q) {
-            const int i = g0 + q * kDenseTeamBlock;
-            if (i >= ie) continue;
-            er = fmax(er, fabs(double(f[i - ib]) - sc[q]));
-            if (x[i]) e += double(d.h[i]) + 0.5 * (sc[q] - double(d.h[i]));
-            x_out[size_t(r) * size_t(n) + size_t(i)] = x[i];
-        }
-    }
+    scratch_fields<kDenseTeamBlock>(d, x, reinterpret_cast<uint16_t*>(blk), ib, ie, [&](int i, double v) {
+        er = fmax(er, fabs(double(f[i - ib]) - v));
+        if (x[i]) e += double(d.h[i]) + 0.5 * (v - double(d.h[i]));
+        x_out[size_t(r) * size_t(n) + size_t(i)] = x[i];
+    });
     for (int o = 32; o > 0; o /= 2) {
         e += __shfl_down(e, o);
         er = fmax(er, __shfl_down(er, o));
