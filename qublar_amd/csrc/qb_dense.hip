@@ -28,6 +28,37 @@ constexpr int kDenseWin = 64;
 constexpr int kRankChunk = 8;
 constexpr int kFieldGroup = 4;   // fields a thread updates together (i, i + block, ...)
 
+// Fields i = g0 + q STRIDE (q < kFieldGroup, i < n) from scratch:
+// h_i + sum_j x_j Q_ji in FP64, j ascending (Q_ji = Q_ij), additions of unset bits
+// skipped; every field's loads of a 16-column chunk in flight together.
+template <int STRIDE>
+__device__ __forceinline__ void scratch_fields_rows(const DevDense& d, const uint8_t* x, int g0, double (&s)[kFieldGroup]) {
+    constexpr int kChunk = 16;
+    const int n = d.n;
+    int col[kFieldGroup];
+#pragma unroll
+    for (int q = 0; q < kFieldGroup; ++q) {
+        col[q] = min(g0 + q * STRIDE, n - 1);
+        s[q] = double(d.h[col[q]]);
+    }
+    for (int j0 = 0; j0 < n; j0 += kChunk) {
+        float v[kFieldGroup][kChunk];
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u)
+#pragma unroll
+            for (int q = 0; q < kFieldGroup; ++q) v[q][u] = d.Q[size_t(min(j0 + u, n - 1)) * size_t(n) + size_t(col[q])];
+#pragma unroll
+        for (int u = 0; u < kChunk; ++u) {
+            const bool set = j0 + u < n && x[min(j0 + u, n - 1)];
+#pragma unroll
+            for (int q = 0; q < kFieldGroup; ++q) {
+                const double nxt = s[q] + double(v[q][u]);
+                s[q] = set ? nxt : s[q];
+            }
+        }
+    }
+}
+
 constexpr int kListBits = 2 * kDenseWin * kDenseWin;   // 16-bit entries in one staging buffer
 
 // The list of the set bits j of x in [p0, p0 + kListBits), less p0, in order; their number.
@@ -89,6 +120,10 @@ __device__ __forceinline__ double add_listed(const DevDense& d, const float* Qp,
 // as many loads are in flight as registers hold (32 twice, and 16 twice where 1,024 threads
 // leave 128 registers). 2,048 bits, 4 workgroups a replica, 32 replicas: 49 us, where the loads
 // of every row, set or not, 16 for four columns each, took 277.
+//
+// FP32 fields only. FP64 fields carry no error, so an anneal with them makes its fields from
+// scratch once, at its end, and every row is read there (scratch_fields_rows): the list in
+// the same kernel costs its windows 2% (4,096 bits, 64 replicas, 500 sweeps: 130.9 -> 133.9 ms).
 template <int THREADS, typename F>
 __device__ __forceinline__ void scratch_fields(const DevDense& d, const uint8_t* x, uint16_t* list, int first,
                                                int last, F&& put) {
@@ -268,18 +303,39 @@ __global__ void __launch_bounds__(kDenseBlock) dense_anneal_kernel(DevDense d, c
         if (recompute_every > 0 && (sweep + 1) % recompute_every == 0) {
             // f = h + Q x from scratch in FP64, j ascending (column i of Q = row i); it reads x and
             // Q only, so fields may change meanwhile. The next window is staged in buffer nbuf.
-            scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk + (nbuf ^ 1) * kDenseWin * kDenseWin), 0,
-                                        n, [&](int i, double v) { f[i] = T(v); });
+            if constexpr (sizeof(T) == 4) {
+                scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk + (nbuf ^ 1) * kDenseWin * kDenseWin),
+                                            0, n, [&](int i, double v) { f[i] = T(v); });
+            } else {
+                for (int g0 = tid; g0 < n; g0 += kFieldGroup * kDenseBlock) {
+                    double sc[kFieldGroup];
+                    scratch_fields_rows<kDenseBlock>(d, x, g0, sc);
+#pragma unroll
+                    for (int q = 0; q < kFieldGroup; ++q)
+                        if (g0 + q * kDenseBlock < n) f[g0 + q * kDenseBlock] = T(sc[q]);
+                }
+            }
             __syncthreads();
         }
     }
     // outputs: spins, the FP64 energy and max |f_carried - f_scratch|
     double e = 0.0, err = 0.0;
-    scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk), 0, n, [&](int i, double v) {
+    auto output = [&](int i, double v) {
         err = fmax(err, fabs(double(f[i]) - v));
         if (x[i]) e += double(d.h[i]) + 0.5 * (v - double(d.h[i]));
         x_out[size_t(blockIdx.x) * size_t(n) + size_t(i)] = x[i];
-    });
+    };
+    if constexpr (sizeof(T) == 4) {
+        scratch_fields<kDenseBlock>(d, x, reinterpret_cast<uint16_t*>(blk), 0, n, output);
+    } else {
+        for (int g0 = tid; g0 < n; g0 += kFieldGroup * kDenseBlock) {
+            double sc[kFieldGroup];
+            scratch_fields_rows<kDenseBlock>(d, x, g0, sc);
+#pragma unroll
+            for (int q = 0; q < kFieldGroup; ++q)
+                if (g0 + q * kDenseBlock < n) output(g0 + q * kDenseBlock, sc[q]);
+        }
+    }
     for (int o = 32; o > 0; o /= 2) {
         e += __shfl_down(e, o);
         err = fmax(err, __shfl_down(err, o));
@@ -678,9 +734,20 @@ __global__ void __launch_bounds__(kDenseTeamBlock) dense_team_kernel(DevDense d,
             // every wave is past the sweep's last window: the fields from scratch in FP64
             // (the next two windows are staged in the two buffers other than the last window's)
             __syncthreads();
-            const int last_buf = ((sweep + 1) * n_win - 1) % 3;
-            scratch_fields<kDenseTeamBlock>(d, x, reinterpret_cast<uint16_t*>(blk + last_buf * kDenseWin * kDenseWin),
-                                            ib, ie, [&](int i, double v) { f[i - ib] = T(v); });
+            if constexpr (sizeof(T) == 4) {
+                const int last_buf = ((sweep + 1) * n_win - 1) % 3;
+                scratch_fields<kDenseTeamBlock>(d, x,
+                                                reinterpret_cast<uint16_t*>(blk + last_buf * kDenseWin * kDenseWin), ib,
+                                                ie, [&](int i, double v) { f[i - ib] = T(v); });
+            } else {
+                for (int g0 = ib + tid; g0 < ie; g0 += kFieldGroup * kDenseTeamBlock) {
+                    double sc[kFieldGroup];
+                    scratch_fields_rows<kDenseTeamBlock>(d, x, g0, sc);
+#pragma unroll
+                    for (int q = 0; q < kFieldGroup; ++q)
+                        if (g0 + q * kDenseTeamBlock < ie) f[g0 + q * kDenseTeamBlock - ib] = T(sc[q]);
+                }
+            }
             __syncthreads();
         }
     }
@@ -688,11 +755,26 @@ __global__ void __launch_bounds__(kDenseTeamBlock) dense_team_kernel(DevDense d,
     if (s_abort) return;
     // outputs: this part's spins, its share of the FP64 energy and of max |f - f_scratch|
     double e = 0.0, er = 0.0;
-    scratch_fields<kDenseTeamBlock>(d, x, reinterpret_cast<uint16_t*>(blk), ib, ie, [&](int i, double v) {
-        er = fmax(er, fabs(double(f[i - ib]) - v));
-        if (x[i]) e += double(d.h[i]) + 0.5 * (v - double(d.h[i]));
-        x_out[size_t(r) * size_t(n) + size_t(i)] = x[i];
-    });
+    if constexpr (sizeof(T) == 4) {
+        scratch_fields<kDenseTeamBlock>(d, x, reinterpret_cast<uint16_t*>(blk), ib, ie, [&](int i, double v) {
+            er = fmax(er, fabs(double(f[i - ib]) - v));
+            if (x[i]) e += double(d.h[i]) + 0.5 * (v - double(d.h[i]));
+            x_out[size_t(r) * size_t(n) + size_t(i)] = x[i];
+        });
+    } else {
+        for (int g0 = ib + tid; g0 < ie; g0 += kFieldGroup * kDenseTeamBlock) {
+            double sc[kFieldGroup];
+            scratch_fields_rows<kDenseTeamBlock>(d, x, g0, sc);
+#pragma unroll
+            for (int q = 0; q < kFieldGroup; ++q) {
+                const int i = g0 + q * kDenseTeamBlock;
+                if (i >= ie) continue;
+                er = fmax(er, fabs(double(f[i - ib]) - sc[q]));
+                if (x[i]) e += double(d.h[i]) + 0.5 * (sc[q] - double(d.h[i]));
+                x_out[size_t(r) * size_t(n) + size_t(i)] = x[i];
+            }
+        }
+    }
     for (int o = 32; o > 0; o /= 2) {
         e += __shfl_down(e, o);
         er = fmax(er, __shfl_down(er, o));

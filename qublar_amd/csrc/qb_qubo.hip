@@ -212,7 +212,7 @@ __global__ void __launch_bounds__(BLOCK) qubo_batch_kernel(DevQuboBatch q, uint3
 // 16th tile of the instance, a lane a bit of it for the four replicas, so a row is read once
 // for all of them in whole lines, eight entries in flight; then a tree over the lanes and the
 // waves. Bound by the latency of the spin words' gathers. 48 instances of 1,000 to 16,384
-// bits, 8 to 32 replicas: 0.24 ms, where a workgroup per job that walked its replicas one
+// bits, 8 to 32 replicas: 0.36 ms, where a workgroup per job that walked its replicas one
 // after the other, a row per lane, took 5.6.
 __global__ void __launch_bounds__(kQuboEnergyBlock) qubo_energy_kernel(DevQuboBatch q, const uint32_t* masks,
                                                                        double* energy) {
