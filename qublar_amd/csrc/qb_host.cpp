@@ -323,7 +323,8 @@ struct qb_problem {
     // workspace
     DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_x16, w_rref,
         w_ref, w_rng, w_energy;
-    size_t ref_entries = 0;   // of the bit-order layout, gaps and padding included
+    size_t ref_entries = 0;    // of the bit-order layout, gaps and padding included
+    int64_t ref_widest = 0;    // the most of them in one window of 64 bits
     int device = 0;   // the device current at creation: its stream, buffers and scratch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ~qb_problem() {
@@ -581,6 +582,8 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
         ref_start[size_t(i) + 1] = (i + 1) % 64 == 0 || i + 1 == n ? (end + 255u) & ~uint64_t(255) : end;
     }
     P->ref_entries = size_t(ref_start.back()) + kRefPad;
+    for (int i = 0; i < n; i += 64)
+        P->ref_widest = std::max(P->ref_widest, int64_t(ref_start[size_t(std::min(i + 64, n))] - ref_start[size_t(i)]));
 
     QB_HIP(hipGetDevice(&P->device));
     QB_HIP(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking));
@@ -1520,8 +1523,8 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
     }
     int launches = 0;
     for (int s0 = 0; s0 < total || launches == 0; s0 += per_launch, ++launches)
-        QB_HIP(launch_ray_ref(P->dev, R, seed_offset, P->w_beta.as<double>(), s0, std::min(total, s0 + per_launch),
-                              P->w_X.as<uint8_t>(), P->w_rref.as<double>(), P->w_rng.as<uint64_t>(), st));
+        QB_HIP(launch_ray_ref(P->dev, P->ref_widest, R, seed_offset, P->w_beta.as<double>(), s0,
+                              std::min(total, s0 + per_launch), P->w_X.as<uint8_t>(), P->w_rref.as<double>(), P->w_rng.as<uint64_t>(), st));
     QB_HIP(hipEventRecord(P->ev1, st));
     // the branches in the group masks of the read-out and energy kernels
     if (n > 0) QB_HIP(launch_pack_states(P->w_X.as<uint8_t>(), R, n, P->dev.pos_bit, P->w_x.as<uint16_t>(), st));

@@ -372,10 +372,11 @@ hipError_t launch_freeze_round(const DevProblem& p, const double* lb, double mar
                                uint8_t* next, unsigned* changed, hipStream_t st);
 // The reference's own float trajectory (anneal_branch): branch b's spins xs[b][bit order]
 // (bytes), residuals rs[b][ray] (FP64) and splitmix64 state sm[b] in global memory; one
-// launch runs sweeps [sweep_begin, sweep_end), the first starting from x = 0.
+// launch runs sweeps [sweep_begin, sweep_end), the first starting from x = 0. `widest`: the most
+// entries of a window in RefLayout.
 hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t entries, hipStream_t st);
-hipError_t launch_ray_ref(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
-                          int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
+hipError_t launch_ray_ref(const DevProblem& p, int64_t widest, int R, uint64_t seed_offset, const double* temp,
+                          int sweep_begin, int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
 // The reference's own integer trajectory (wising::anneal), one wave per replica with its
 // state in LDS (n_pad * 5 bytes; four replicas per workgroup while that fits), or in global
 // memory when one replica's state exceeds kRefLdsLimit: temp[sweep] is the temperature,

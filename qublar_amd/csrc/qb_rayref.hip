@@ -22,7 +22,7 @@ using f64x2 = double __attribute__((ext_vector_type(2)));
 
 constexpr int kQuads = 3;               // four entries of a lane each, in flight
 constexpr int kBatch = 256 * kQuads;    // entries of a batch
-constexpr int kPass = 5 * kBatch;       // terms of one pass in LDS
+constexpr int kPassBatches = 5;         // batches of one pass at most, its terms in LDS
 constexpr int kTail = 16;               // terms a lane reads ahead of its sum
 constexpr int kNb = kRefNb;             // neighbours of a bit held in registers; more are read in turn
 static_assert(2 * kBatch <= kRefPad && kNb == 8);
@@ -61,9 +61,10 @@ __device__ __forceinline__ double flip_sign(double v, uint32_t bit) {
 template <bool LDS_X>
 __global__ void __launch_bounds__(64) ray_ref_kernel(DevProblem p, uint64_t seed_offset, const double* temp,
                                                       int sweep_begin, int sweep_end, uint8_t* xs, double* rs,
-                                                      uint64_t* sm) {
-    __shared__ __align__(16) double terms[kPass + 2 * kTail];
-    extern __shared__ uint64_t xw[];   // LDS_X: bit i of the branch is bit i % 64 of word i / 64
+                                                      uint64_t* sm, int pass) {
+    extern __shared__ __align__(16) double terms[];   // pass terms, and what a lane reads past them
+    // LDS_X: bit i of the branch is bit i % 64 of word i / 64
+    uint64_t* xw = reinterpret_cast<uint64_t*>(terms + pass + 2 * kTail);
     const int lane = int(threadIdx.x), b = int(blockIdx.x);
     const int n = p.n, n_win = (n + 63) / 64;
     uint8_t* x = xs + size_t(b) * size_t(n);
@@ -179,7 +180,7 @@ __global__ void __launch_bounds__(64) ray_ref_kernel(DevProblem p, uint64_t seed
             uint64_t from = base;
             for (;;) {
                 for (uint64_t p0 = from, p1; p0 < end; p0 = p1) {
-                    p1 = end - p0 > kPass ? p0 + kPass : end;
+                    p1 = end - p0 > uint64_t(pass) ? p0 + uint64_t(pass) : end;
                     if (held != p0) {   // in the loop's order, so that its waits fit both
 #pragma unroll
                         for (int v = 0; v < kQuads; ++v) load_rays(v, p0);
@@ -204,34 +205,36 @@ __global__ void __launch_bounds__(64) ray_ref_kernel(DevProblem p, uint64_t seed
 #pragma unroll
                         for (int v = 0; v < kQuads; ++v) {
                             __builtin_amdgcn_sched_barrier(0);
-                            // a is a float's value, so 0.5 a a is exact and the fused add rounds
-                            // as the separate one does; four entries side by side, as the wave
-                            // has its SIMD to itself and each step's result takes a while
-                            double ad[4], t[4];
+                            if (int(p1 - g) > 256 * v) {   // the batch's last blocks may be empty
+                                // a is a float's value, so 0.5 a a is exact and the fused add rounds
+                                // as the separate one does; four entries side by side, as the wave
+                                // has its SIMD to itself and each step's result takes a while
+                                double ad[4], t[4];
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) ad[u] = double(a[v][u]);
-                            uint32_t neg[4];
+                                for (int u = 0; u < 4; ++u) ad[u] = double(a[v][u]);
+                                uint32_t neg[4];
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) neg[u] = uint32_t(xmask >> ((own[v] >> (8 * u)) & 63u)) << 31;
-                            __builtin_amdgcn_sched_barrier(0);
+                                for (int u = 0; u < 4; ++u) neg[u] = uint32_t(xmask >> ((own[v] >> (8 * u)) & 63u)) << 31;
+                                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u)
-                                ad[u] = __hiloint2double(__double2hiint(ad[u]) ^ int(neg[u]), __double2loint(ad[u]));
-                            __builtin_amdgcn_sched_barrier(0);
+                                for (int u = 0; u < 4; ++u)
+                                    ad[u] = __hiloint2double(__double2hiint(ad[u]) ^ int(neg[u]), __double2loint(ad[u]));
+                                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) t[u] = rv[v][u] * ad[u];
-                            double half[4];
+                                for (int u = 0; u < 4; ++u) t[u] = rv[v][u] * ad[u];
+                                double half[4];
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) half[u] = 0.5 * ad[u];
-                            __builtin_amdgcn_sched_barrier(0);
+                                for (int u = 0; u < 4; ++u) half[u] = 0.5 * ad[u];
+                                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) t[u] = __builtin_fma(half[u], ad[u], t[u]);
-                            __builtin_amdgcn_sched_barrier(0);
+                                for (int u = 0; u < 4; ++u) t[u] = __builtin_fma(half[u], ad[u], t[u]);
+                                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) t[u] *= w[v][u / 2][u % 2];
-                            __builtin_amdgcn_sched_barrier(0);
+                                for (int u = 0; u < 4; ++u) t[u] *= w[v][u / 2][u % 2];
+                                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                            for (int u = 0; u < 4; ++u) terms[int(g - p0) + 256 * v + 64 * u + lane] = t[u];
+                                for (int u = 0; u < 4; ++u) terms[int(g - p0) + 256 * v + 64 * u + lane] = t[u];
+                            }
                             __builtin_amdgcn_sched_barrier(0);
                             load_residuals(v);
                             load_rays(v, then + kBatch);
@@ -383,14 +386,20 @@ hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t en
     return hipGetLastError();
 }
 
-hipError_t launch_ray_ref(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
+hipError_t launch_ray_ref(const DevProblem& p, int64_t widest, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
                           int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st) {
+    // a pass holds the widest window where it can: with fewer terms in LDS more branches share a
+    // CU (4,096 branches of 100 bits and 500 entries, 20 sweeps at T = 20: 22.6 ms with five batches, 22.1
+    // with one; there a CU holds eight waves and their instructions bound it)
+    const int pass = kBatch * int(std::clamp<int64_t>((widest + kBatch - 1) / kBatch, 1, kPassBatches));
+    const size_t terms = sizeof(double) * size_t(pass + 2 * kTail);
     const size_t mask = sizeof(uint64_t) * ((size_t(p.n) + 63) / 64);
-    // 64 KiB with the terms: 260,096 bits
-    if (mask <= 32768 - sizeof(double) * 2 * kTail)
-        ray_ref_kernel<true><<<unsigned(R), 64, mask, st>>>(p, seed_offset, temp, sweep_begin, sweep_end, xs, rs, sm);
+    if (mask <= 32768 - sizeof(double) * 2 * kTail)   // 260,096 bits; within 64 KiB with the terms
+        ray_ref_kernel<true>
+            <<<unsigned(R), 64, terms + mask, st>>>(p, seed_offset, temp, sweep_begin, sweep_end, xs, rs, sm, pass);
     else
-        ray_ref_kernel<false><<<unsigned(R), 64, 0, st>>>(p, seed_offset, temp, sweep_begin, sweep_end, xs, rs, sm);
+        ray_ref_kernel<false>
+            <<<unsigned(R), 64, terms, st>>>(p, seed_offset, temp, sweep_begin, sweep_end, xs, rs, sm, pass);
     return hipGetLastError();
 }
 
