@@ -223,9 +223,13 @@ __device__ __forceinline__ double wave_sum(double v) {
 
 // Z and the weighted sums of the low and thread bits of every block (kRoiSums values: Z, the
 // low bits', the thread bits'). PROD: a group's weights as products of 6 exponentials --
-// the host checks that no factor can leave the range of a double; every product is itself a
-// state's weight (at most 1, up to the carried energies' rounding), so a weight that
-// underflows is below 2^-1074 e^600 of Z. Otherwise one exponential per state.
+// made and summed relative to its first state's, which the host's check holds between e^-600
+// and e^600, so none of them leaves a double's ordinary range; each sum is then scaled by the
+// first state's weight, in two factors of its root, as that weight itself may underflow where
+// the group's other states have weights a marginal is made of. A sum thus keeps its accuracy
+// down to a double's smallest ordinary value, as one exponential per state does (the other form).
+// The scaling is 12 multiplications in about 320 instructions a group (a call: 26 bits 0.133 ms, 32
+// bits 2.13 ms, both as without it).
 template <int B, bool PROD>
 __global__ void __launch_bounds__(kRoiBlock) roi_sum_kernel(int n, const double* h, const double* Js, double beta,
                                                             const double* e_min, const double* factors, double* blk) {
@@ -245,7 +249,7 @@ __global__ void __launch_bounds__(kRoiBlock) roi_sum_kernel(int n, const double*
         const unsigned gray = t > 0 ? w.step(s, t) : 0u;
         double W[kRoiStates];
         if constexpr (PROD) {
-            W[0] = exp(-beta * (w.e - e_ref));
+            W[0] = 1.0;
 #pragma unroll
             for (int a = 0; a < kRoiGroupBits; ++a) {
                 double T[kRoiStates / 2];
@@ -262,6 +266,8 @@ __global__ void __launch_bounds__(kRoiBlock) roi_sum_kernel(int n, const double*
 #pragma unroll
             for (int q = 0; q < kRoiStates; ++q) W[q] = exp(-beta * (W[q] - e_ref));
         }
+        const double root = PROD ? exp(-0.5 * beta * (w.e - e_ref)) : 1.0;
+        auto scaled = [&](double v) { return PROD ? v * root * root : v; };
         // pairwise over the group's bits: the odd half of each level is that bit's weight
 #pragma unroll
         for (int a = 0; a < kRoiGroupBits; ++a) {
@@ -274,9 +280,9 @@ __global__ void __launch_bounds__(kRoiBlock) roi_sum_kernel(int n, const double*
                     odd += W[2 * q + 1];
                     W[q] = W[2 * q] + W[2 * q + 1];
                 }
-            m[a] += odd;
+            m[a] += scaled(odd);
         }
-        const double zg = W[0];
+        const double zg = scaled(W[0]);
         z += zg;
 #pragma unroll
         for (int j = kRoiGroupBits; j < L; ++j) m[j] += ((gray >> (j - kRoiGroupBits)) & 1u) ? zg : 0.0;
