@@ -488,7 +488,7 @@ typedef struct {
     double kernel_ms;         /* annealing kernels only, HIP events */
     int launches;
     int replica_block;        /* the replica block the run used */
-    int jobs;
+    int jobs;                 /* replica blocks run, a long instance's in halves at replica_block 4 */
     int block;                /* the threads per workgroup it used */
     double spin_updates;      /* sum over instances of replicas x sweeps x n_k */
     int graph_replayed;       /* 1 when the anneal replayed a graph recorded by an earlier call */

@@ -2092,7 +2092,6 @@ struct qb_qubo_batch {
         std::vector<QuboJob> host;    // instance order
         std::vector<int32_t> first;   // per instance: its first job in instance order
         int64_t mask_words = 0;
-        int blocks = 0;   // replica blocks; long ones are two jobs
     };
     std::map<int, std::unique_ptr<Jobs>> jobs;   // by replica block
     DevBuf w_mask, w_beta, w_queue, w_energy;
@@ -2372,7 +2371,6 @@ static int qubo_jobs_for(qb_qubo_batch* B, int rb, const qb_qubo_batch::Jobs** o
     int64_t words = 0;
     for (int k = 0; k < B->n_inst; ++k) {
         Jb->first.push_back(int32_t(Jb->host.size()));
-        Jb->blocks += (B->replicas[size_t(k)] + rb - 1) / rb;
         for (int r0 = 0; r0 < B->replicas[size_t(k)]; r0 += size[size_t(k)]) {
             QuboJob j{};
             j.instance = k;
@@ -2616,7 +2614,7 @@ extern "C" int qb_qubo_batch_anneal(qb_qubo_batch* B, const qb_schedule* s, cons
         rep->launches = launches;
         rep->replica_block = rb;
         rep->block = block;
-        rep->jobs = Jb->blocks;
+        rep->jobs = int(Jb->host.size());
         rep->graph_replayed = replayed ? 1 : 0;
         double upd = 0.0;
         for (int k = 0; k < B->n_inst; ++k) upd += double(B->replicas[size_t(k)]) * double(B->n_bits[size_t(k)]);
