@@ -305,7 +305,7 @@ struct qb_problem {
     int64_t device_bytes = 0;
     std::vector<int32_t> pos_bit, cls_ptr;
     DevBuf b_cls, b_pos, b_col, b_ent, b_nbp, b_nb, b_nbbit, b_lin, b_d, b_w, b_rtp, b_rt, b_seq, b_dbit, b_dkey,
-        b_lbeg, b_lnb, b_bitpos, b_refst;
+        b_lbeg, b_lnb, b_bitpos;
     std::vector<int32_t> light_begin;   // host copy: each class's first light position
     std::vector<int32_t> col_ptr, nb_ptr;   // host copies, position space
     std::vector<uint8_t> seq_update;
@@ -323,8 +323,7 @@ struct qb_problem {
     // workspace
     DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_x16, w_rref,
         w_ref, w_rng, w_energy;
-    size_t ref_entries = 0;    // of the bit-order layout, gaps and padding included
-    int64_t ref_widest = 0;    // the most of them in one window of 64 bits
+    int64_t ref_widest = 0;    // the most entries that one window of 64 bits has in dev.ref
     int device = 0;   // the device current at creation: its stream, buffers and scratch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ~qb_problem() {
@@ -576,14 +575,6 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
     std::vector<BitEnt> rt(static_cast<size_t>(nnz));
     for (size_t q = 0; q < rt.size(); ++q) rt[q] = BitEnt{pos_of[size_t(rt_bit[q])], rt_a[q]};
     std::vector<double> dv(desc->d, desc->d + nr), wv(desc->w, desc->w + nr);
-    std::vector<uint64_t> ref_start(size_t(n) + 1, 0);
-    for (int i = 0; i < n; ++i) {
-        const uint64_t end = ref_start[size_t(i)] + uint64_t(desc->row_ptr[i + 1] - desc->row_ptr[i]);
-        ref_start[size_t(i) + 1] = (i + 1) % 64 == 0 || i + 1 == n ? (end + 255u) & ~uint64_t(255) : end;
-    }
-    P->ref_entries = size_t(ref_start.back()) + kRefPad;
-    for (int i = 0; i < n; i += 64)
-        P->ref_widest = std::max(P->ref_widest, int64_t(ref_start[size_t(std::min(i + 64, n))] - ref_start[size_t(i)]));
 
     QB_HIP(hipGetDevice(&P->device));
     QB_HIP(hipStreamCreateWithFlags(&P->stream, hipStreamNonBlocking));
@@ -597,8 +588,7 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
         (rc = P->b_col.upload(col_ptr, st)) || (rc = P->b_ent.upload(ent, st)) || (rc = P->b_nbp.upload(nb_ptr, st)) ||
         (rc = P->b_nb.upload(nb, st)) || (rc = P->b_nbbit.upload(nb_bit, st)) || (rc = P->b_lin.upload(lin, st)) ||
         (rc = P->b_d.upload(dv, st)) || (rc = P->b_w.upload(wv, st)) || (rc = P->b_rtp.upload(rt_ptr, st)) ||
-        (rc = P->b_rt.upload(rt, st)) || (rc = P->b_bitpos.upload(pos_of, st)) ||
-        (rc = P->b_refst.upload(ref_start, st)))
+        (rc = P->b_rt.upload(rt, st)) || (rc = P->b_bitpos.upload(pos_of, st)))
         return rc;
     QB_HIP(hipStreamSynchronize(st));
     P->col_ptr = col_ptr;
@@ -626,7 +616,6 @@ extern "C" int qb_problem_create(const qb_problem_desc* desc, qb_problem** out) 
     D.bit_pos = P->b_bitpos.as<int32_t>();
     D.col_ptr = P->b_col.as<int32_t>();
     D.ent = P->b_ent.as<RayEnt>();
-    D.ref_start = P->b_refst.as<uint64_t>();
     D.nb_ptr = P->b_nbp.as<int32_t>();
     D.nb = P->b_nb.as<int32_t>();
     D.nb_bit = P->b_nbbit.as<int32_t>();
@@ -1457,6 +1446,45 @@ extern "C" int qb_stage_sweeps(const qb_stage* S, int* sweeps) {
 // leaves the split to the library (about a second at a few branches of the muon QUBO).
 constexpr double kRefFloatUpdatesPerLaunch = 33554432.0;
 
+// The problem laid out in bit order (dev.ref), on the first anneal that reads it.
+static int ref_layout_for(qb_problem* P) {
+    if (P->dev.ref.w) return QB_OK;
+    const int n = P->n;
+    std::vector<uint64_t> start(size_t(n) + 1, 0);   // each bit's first entry, and behind the last bit
+    for (int p = 0; p < n; ++p)
+        start[size_t(P->pos_bit[size_t(p)]) + 1] = uint64_t(P->col_ptr[size_t(p) + 1] - P->col_ptr[size_t(p)]);
+    for (int i = 0; i < n; ++i) {
+        const uint64_t end = start[size_t(i)] + start[size_t(i) + 1];
+        start[size_t(i) + 1] = (i + 1) % 64 == 0 || i + 1 == n ? (end + 255u) & ~uint64_t(255) : end;
+    }
+    int64_t widest = 0;
+    for (int i = 0; i < n; i += 64)
+        widest = std::max(widest, int64_t(start[size_t(std::min(i + 64, n))] - start[size_t(i)]));
+    const size_t entries = size_t(start.back()) + kRefPad;
+    const size_t per_entry = sizeof(double) + sizeof(uint32_t) + sizeof(float) + 1;
+    const size_t per_bit = sizeof(RefBit) + sizeof(RefBase) + sizeof(int32_t) * kRefNb;
+    DevBuf d_start;
+    int rc;
+    if ((rc = P->w_ref.reserve(per_entry * entries + per_bit * size_t(n))) || (rc = d_start.upload(start, P->stream)))
+        return rc;
+    char* at = P->w_ref.as<char>();
+    RefLayout to;
+    to.w = reinterpret_cast<double*>(at);
+    to.bit = reinterpret_cast<RefBit*>(at += sizeof(double) * entries);
+    to.base = reinterpret_cast<RefBase*>(at += sizeof(RefBit) * size_t(n));
+    to.nb = reinterpret_cast<int32_t*>(at += sizeof(RefBase) * size_t(n));
+    to.ray = reinterpret_cast<uint32_t*>(at += sizeof(int32_t) * kRefNb * size_t(n));
+    to.a = reinterpret_cast<float*>(at += sizeof(uint32_t) * entries);
+    to.own = reinterpret_cast<uint8_t*>(at + sizeof(float) * entries);
+    DevProblem with_start = P->dev;
+    with_start.ref_start = d_start.as<uint64_t>();
+    QB_HIP(launch_ref_layout(with_start, to, entries, P->stream));
+    QB_HIP(hipStreamSynchronize(P->stream));
+    P->dev.ref = to;
+    P->ref_widest = widest;
+    return QB_OK;
+}
+
 extern "C" int qb_anneal_branches_reference(qb_problem* P, const qb_schedule* s, int n_branches, uint64_t seed_offset,
                                            uint8_t* branches, float* p_void, uint8_t* tri, float* certainty,
                                            double* energy, qb_report* rep) {
@@ -1481,12 +1509,8 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
         per_launch = int(std::clamp(kRefFloatUpdatesPerLaunch / (double(R) * double(std::max(n, 1))), 1.0,
                                     double(std::max(total, 1))));
     const int n_groups = (R + kGroup - 1) / kGroup;
-    const size_t n_ref = P->ref_entries;
-    const size_t per_entry = sizeof(double) + sizeof(uint32_t) + sizeof(float) + 1;
-    const size_t per_bit = sizeof(RefBit) + sizeof(RefBase) + sizeof(int32_t) * kRefNb;
     const int n_part = ray_energy_blocks(P->dev);
-    if ((rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
-        (rc = P->w_ref.reserve(per_entry * n_ref + per_bit * size_t(n))) ||
+    if ((rc = ref_layout_for(P)) || (rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
         (rc = P->w_rref.reserve(sizeof(double) * size_t(R) * size_t(std::max(nr, 1)))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
         (rc = P->w_x.reserve(sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
@@ -1508,19 +1532,6 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(P->w_beta.p, temp.data(), sizeof(double) * temp.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(P->ev0, st));
-    if (!P->dev.ref.w) {
-        char* at = P->w_ref.as<char>();
-        RefLayout to;
-        to.w = reinterpret_cast<double*>(at);
-        to.bit = reinterpret_cast<RefBit*>(at += sizeof(double) * n_ref);
-        to.base = reinterpret_cast<RefBase*>(at += sizeof(RefBit) * size_t(n));
-        to.nb = reinterpret_cast<int32_t*>(at += sizeof(RefBase) * size_t(n));
-        to.ray = reinterpret_cast<uint32_t*>(at += sizeof(int32_t) * kRefNb * size_t(n));
-        to.a = reinterpret_cast<float*>(at += sizeof(uint32_t) * n_ref);
-        to.own = reinterpret_cast<uint8_t*>(at + sizeof(float) * n_ref);
-        QB_HIP(launch_ref_layout(P->dev, to, n_ref, st));
-        P->dev.ref = to;
-    }
     int launches = 0;
     for (int s0 = 0; s0 < total || launches == 0; s0 += per_launch, ++launches)
         QB_HIP(launch_ray_ref(P->dev, P->ref_widest, R, seed_offset, P->w_beta.as<double>(), s0,

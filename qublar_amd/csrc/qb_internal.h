@@ -89,7 +89,7 @@ struct DevProblem {
     // CSR order (-1 past its last).
     const int32_t* light_begin;
     const int32_t* light_nb;
-    const uint64_t* ref_start;   // the first entry of each bit in ref, and behind the last bit
+    const uint64_t* ref_start;   // the first entry of each bit in ref, and behind the last bit (for its layout)
     RefLayout ref;               // laid out on the first anneal on the reference's own trajectory
     double lambda;
 };
