@@ -87,6 +87,14 @@ static int device_props(hipDeviceProp_t& prop) {
     return QB_OK;
 }
 
+// Compute units of the current device.
+static int device_cus(int& cus) {
+    int dev = 0;
+    QB_HIP(hipGetDevice(&dev));
+    QB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+    return QB_OK;
+}
+
 extern "C" int qb_get_device_info(qb_device_info* out) {
     if (!out) return fail(QB_E_ARG, "qb_get_device_info: null output");
     hipDeviceProp_t prop;
@@ -1715,7 +1723,7 @@ struct qb_graph {
     DevGraph dev{};
     qb_plan plan{};
     bool lds_state = false;
-    std::vector<int32_t> pos_bit, cls_ptr;
+    std::vector<int32_t> pos_bit, cls_ptr, nb_ptr;
     DevBuf b_cls, b_pos, b_nbp, b_nb, b_nw, b_f0, b_eu, b_ev, b_ew, b_bitpos, b_orows, b_prows, b_ostart, b_band, b_steps;
     int cus = 0;   // compute units of its device
     DevBuf w_s, w_f, w_e, w_sout, w_beta, w_X, w_out, w_rng;
@@ -1868,6 +1876,7 @@ extern "C" int qb_graph_create(const qb_graph_desc* d, int force_global, qb_grap
         nb_ptr[size_t(p) + 1] = int32_t(q);
         f0[size_t(p)] = int32_t(acc);
     }
+    G->nb_ptr = nb_ptr;
     const int64_t lds_need = int64_t(G->plan.n_pad) * 5;
     G->lds_state = !force_global && G->plan.n_pad <= int_lds_capacity_spins() && lds_need <= 64 * 1024;
     G->plan.shared_state = G->lds_state ? 1 : 0;
@@ -1877,43 +1886,15 @@ extern "C" int qb_graph_create(const qb_graph_desc* d, int force_global, qb_grap
     hipStream_t st = G->stream;
     std::vector<int32_t> eu(d->eu, d->eu + m), ev(d->ev, d->ev + m), ewv(d->ew, d->ew + m);
     int rc;
-    hipDeviceProp_t prop;
-    if ((rc = device_props(prop))) return rc;
-    G->cus = prop.multiProcessorCount;
-    // rows of 16-bit words where one magnitude serves every coupling
-    const bool one_weight = n <= 32768 && m > 0 && 2 * m <= int64_t(INT32_MAX) && G->plan.max_w < (int64_t(1) << 30) &&
-                            std::all_of(w.begin(), w.end(), [&](int32_t v) { return v != 0 && std::abs(int64_t(v)) == G->plan.max_w; });
-    if (one_weight) {
-        std::vector<uint16_t> orows(size_t(2 * m)), prows(size_t(2 * m));
-        std::vector<int32_t> ostart(row.begin(), row.end());
-        for (size_t q = 0; q < orows.size(); ++q) {
-            orows[q] = uint16_t(col[q] | (w[q] < 0 ? 0x8000 : 0));
-            prows[q] = uint16_t(nb[q] | (nw[q] < 0 ? 0x8000 : 0));
-        }
-        std::vector<uint64_t> band(static_cast<size_t>(n), 0u);
-        for (int i = 0; i < n; ++i)
-            for (int64_t k = row[size_t(i)]; k < row[size_t(i) + 1]; ++k) {
-                const int back = i - col[size_t(k)];
-                if (back >= 1 && back <= 64) band[size_t(i)] |= uint64_t(1) << (64 - back);
-            }
-        std::vector<int32_t> steps{0};   // every class in equal steps
-        for (int c = 0; c < K; ++c) {
-            const int c0 = G->cls_ptr[size_t(c)], size = G->cls_ptr[size_t(c) + 1] - c0;
-            const int parts = (size + kWideDraws - 1) / kWideDraws;
-            for (int q = 1; q <= parts; ++q) steps.push_back(c0 + int(int64_t(size) * q / parts));
-        }
-        if ((rc = G->b_steps.upload(steps, st)) || (rc = G->b_band.upload(band, st)) || (rc = G->b_orows.upload(orows, st)) || (rc = G->b_prows.upload(prows, st)) ||
-            (rc = G->b_ostart.upload(ostart, st)))
-            return rc;
-        QB_HIP(hipStreamSynchronize(st));
-        G->dev.orows = G->b_orows.as<uint16_t>();
-        G->dev.prows = G->b_prows.as<uint16_t>();
-        G->dev.ostart = G->b_ostart.as<int32_t>();
-        G->dev.band = G->b_band.as<uint64_t>();
-        G->dev.steps = G->b_steps.as<int32_t>();
-        G->dev.n_steps = int(steps.size()) - 1;
+    if ((rc = device_cus(G->cus))) return rc;
+    // rows of 16-bit words where one magnitude serves every coupling, laid out by the first
+    // anneal that reads them (position_rows, bit_rows)
+    if (n <= 32768 && m > 0 && 2 * m <= int64_t(INT32_MAX) && G->plan.max_w < (int64_t(1) << 30) &&
+        G->plan.w_min == G->plan.max_w && std::all_of(d->ew, d->ew + m, [](int32_t v) { return v != 0; })) {
         G->dev.w0 = int(G->plan.max_w);
         G->dev.m_dir = int(2 * m);
+        for (int c = 0; c < K; ++c)
+            G->dev.n_steps += (G->cls_ptr[size_t(c) + 1] - G->cls_ptr[size_t(c)] + kWideDraws - 1) / kWideDraws;
     }
     if ((rc = G->b_cls.upload(G->cls_ptr, st)) || (rc = G->b_pos.upload(G->pos_bit, st)) ||
         (rc = G->b_nbp.upload(nb_ptr, st)) || (rc = G->b_nb.upload(nb, st)) || (rc = G->b_nw.upload(nw, st)) ||
@@ -1958,6 +1939,46 @@ extern "C" int qb_graph_colouring(const qb_graph* g, int32_t* order, int32_t* cl
     return QB_OK;
 }
 
+// The 16-bit rows in position order, and the classes in equal steps, on the first anneal that
+// reads them.
+static int position_rows(qb_graph* G) {
+    if (G->dev.prows) return QB_OK;
+    std::vector<int32_t> steps{0};
+    for (int c = 0; c < G->plan.n_classes; ++c) {
+        const int c0 = G->cls_ptr[size_t(c)], size = G->cls_ptr[size_t(c) + 1] - c0;
+        const int parts = (size + kWideDraws - 1) / kWideDraws;
+        for (int q = 1; q <= parts; ++q) steps.push_back(c0 + int(int64_t(size) * q / parts));
+    }
+    int rc;
+    if ((rc = G->b_prows.reserve(sizeof(uint16_t) * size_t(G->dev.m_dir))) || (rc = G->b_steps.upload(steps, G->stream)))
+        return rc;
+    QB_HIP(launch_position_rows(G->dev, G->b_prows.as<uint16_t>(), G->stream));
+    QB_HIP(hipStreamSynchronize(G->stream));
+    G->dev.steps = G->b_steps.as<int32_t>();
+    G->dev.prows = G->b_prows.as<uint16_t>();
+    return QB_OK;
+}
+
+// The 16-bit rows in original bit order with their starts and bands, on the first such anneal.
+static int bit_rows(qb_graph* G) {
+    if (G->dev.orows) return QB_OK;
+    const int n = G->plan.n;
+    std::vector<int32_t> start(size_t(n) + 1, 0);
+    for (int p = 0; p < n; ++p)
+        start[size_t(G->pos_bit[size_t(p)]) + 1] = G->nb_ptr[size_t(p) + 1] - G->nb_ptr[size_t(p)];
+    for (int i = 0; i < n; ++i) start[size_t(i) + 1] += start[size_t(i)];
+    int rc;
+    if ((rc = G->b_orows.reserve(sizeof(uint16_t) * size_t(G->dev.m_dir))) ||
+        (rc = G->b_band.reserve(sizeof(uint64_t) * size_t(n))) || (rc = G->b_ostart.upload(start, G->stream)))
+        return rc;
+    G->dev.ostart = G->b_ostart.as<int32_t>();
+    G->dev.band = G->b_band.as<uint64_t>();
+    QB_HIP(launch_bit_rows(G->dev, G->b_orows.as<uint16_t>(), G->b_band.as<uint64_t>(), G->stream));
+    QB_HIP(hipStreamSynchronize(G->stream));
+    G->dev.orows = G->b_orows.as<uint16_t>();
+    return QB_OK;
+}
+
 extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_base, int R, double updates_per_launch,
                             int8_t* s_out, int64_t* energy_out, qb_batch_report* rep) {
     if (!G) return fail(QB_E_ARG, "qb_run_batch: null graph");
@@ -1971,6 +1992,9 @@ extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_bas
     if ((rc = G->w_s.reserve(cells)) || (rc = G->w_f.reserve(cells * 4)) || (rc = G->w_e.reserve(sizeof(long long) * size_t(R))) ||
         (rc = G->w_sout.reserve(cells)) || (rc = G->w_beta.reserve(sizeof(double) * size_t(total))))
         return rc;
+    // force_global keeps the state in global memory
+    const IntShape sh = G->lds_state ? int_shape(G->dev, R, G->cus) : IntShape{kIntSweep, 0};
+    if (sh.kind != kIntSweep && (rc = position_rows(G))) return rc;
     const std::vector<double> beta = betas_of(*b);
     hipStream_t st = G->stream;
     int chunk = int(std::floor(updates_per_launch / (double(R) * double(n))));
@@ -1979,8 +2003,6 @@ extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_bas
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(G->w_beta.p, beta.data(), sizeof(double) * beta.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(G->ev0, st));
-    // force_global keeps the state in global memory
-    const IntShape sh = G->lds_state ? int_shape(G->dev, R, G->cus) : IntShape{kIntSweep, 0};
     int launches = 0;
     for (int sb = 0; sb < total; sb += chunk) {
         const int se = std::min(total, sb + chunk), init = sb == 0 ? 1 : 0;
@@ -2026,6 +2048,9 @@ extern "C" int qb_run_batch_reference(qb_graph* G, const qb_schedule* b, uint64_
         (rc = G->w_e.reserve(sizeof(long long) * size_t(R))) || (rc = G->w_rng.reserve(sizeof(uint64_t) * size_t(R))) ||
         (rc = G->w_sout.reserve(cells)) || (rc = G->w_beta.reserve(sizeof(double) * size_t(total))))
         return rc;
+    bool lds_rows = false;
+    const int waves = int_ref_rows_waves(G->dev, R, G->cus, &lds_rows);
+    if (waves > 0 && (rc = bit_rows(G))) return rc;
     // the temperature of every sweep by the reference's expression (src/ising_weighted.hpp:255-258)
     std::vector<double> temp(static_cast<size_t>(total));
     for (int sweep = 0; sweep < total; ++sweep) {
@@ -2039,8 +2064,6 @@ extern "C" int qb_run_batch_reference(qb_graph* G, const qb_schedule* b, uint64_
     const auto t0 = std::chrono::steady_clock::now();
     QB_HIP(hipMemcpyAsync(G->w_beta.p, temp.data(), sizeof(double) * temp.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(G->ev0, st));
-    bool lds_rows = false;
-    const int waves = int_ref_rows_waves(G->dev, R, G->cus, &lds_rows);
     int launches = 0;
     for (int sb = 0; sb < total; sb += chunk) {
         const int se = std::min(total, sb + chunk), init = sb == 0 ? 1 : 0;

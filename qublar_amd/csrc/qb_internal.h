@@ -208,9 +208,10 @@ struct DevGraph {
     const int32_t* nw;
     const int32_t* f0;      // fields of the all-zero assignment
     const int32_t* bit_pos; // original bit -> position
-    // Where every coupling has the magnitude w0 and n <= 32768 (null otherwise): the rows as
-    // 16-bit words, neighbour | sign << 15, padded to whole 32-bit words -- orows in original
-    // bit order with its row starts, prows in position order (starts nb_ptr).
+    // Where every coupling has the magnitude w0 and n <= 32768 (w0 = 0 otherwise): the rows as
+    // 16-bit words, neighbour | sign << 15 -- orows in original bit order with its row starts
+    // and bands, prows in position order (starts nb_ptr) with the steps; each null until the
+    // first anneal that reads it.
     const uint16_t* orows;
     const uint16_t* prows;
     const int32_t* ostart;
@@ -387,6 +388,9 @@ bool int_ref_in_lds(const DevGraph& g);
 hipError_t launch_int_ref(const DevGraph& g, int R, uint64_t seed_base, const double* temp, int sweep_begin,
                           int sweep_end, int init, int8_t* s_state, int32_t* f_state, uint64_t* rng,
                           long long* energy, hipStream_t st);
+// The 16-bit rows: prows, or orows and band (g.ostart set).
+hipError_t launch_position_rows(const DevGraph& g, uint16_t* prows, hipStream_t st);
+hipError_t launch_bit_rows(const DevGraph& g, uint16_t* orows, uint64_t* band, hipStream_t st);
 // The same trajectory on 16-bit rows (in LDS or not), `waves` replicas per workgroup
 // (int_ref_rows_waves > 0).
 int int_ref_rows_waves(const DevGraph& g, int R, int cus, bool* lds_rows);

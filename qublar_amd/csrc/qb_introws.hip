@@ -59,7 +59,39 @@ __device__ __forceinline__ void rows_add(const uint16_t* rows, uint64_t m, int l
     }
 }
 
+// The rows in position order.
+__global__ void __launch_bounds__(256) position_rows_kernel(DevGraph g, uint16_t* prows) {
+    for (int q = int(blockIdx.x) * 256 + int(threadIdx.x); q < g.m_dir; q += int(gridDim.x) * 256)
+        prows[q] = uint16_t(g.nb[q] | (g.nw[q] < 0 ? 0x8000 : 0));
+}
+
+// The rows in original bit order, one wave a bit, and each bit's band.
+__global__ void __launch_bounds__(256) bit_rows_kernel(DevGraph g, uint16_t* orows, uint64_t* band) {
+    const int i = int(blockIdx.x) * 4 + int(threadIdx.x) / 64, lane = int(threadIdx.x) % 64;
+    if (i >= g.n) return;   // the whole wave
+    const int p = g.bit_pos[i], q0 = g.nb_ptr[p], len = g.nb_ptr[p + 1] - q0;
+    uint16_t* row = orows + g.ostart[i];
+    uint64_t m = 0;
+    for (int k = lane; k < len; k += 64) {
+        const int j = g.pos_bit[g.nb[q0 + k]], back = i - j;
+        row[k] = uint16_t(j | (g.nw[q0 + k] < 0 ? 0x8000 : 0));
+        if (back >= 1 && back <= 64) m |= uint64_t(1) << (64 - back);
+    }
+    for (int o = 32; o > 0; o >>= 1) m |= uint64_t(__shfl_xor((unsigned long long)m, o));
+    if (lane == 0) band[i] = m;
+}
+
 }  // namespace
+
+hipError_t launch_position_rows(const DevGraph& g, uint16_t* prows, hipStream_t st) {
+    position_rows_kernel<<<unsigned(std::min(2048, (g.m_dir + 255) / 256)), 256, 0, st>>>(g, prows);
+    return hipGetLastError();
+}
+
+hipError_t launch_bit_rows(const DevGraph& g, uint16_t* orows, uint64_t* band, hipStream_t st) {
+    bit_rows_kernel<<<unsigned((g.n + 3) / 4), 256, 0, st>>>(g, orows, band);
+    return hipGetLastError();
+}
 
 // ---- the reference's own trajectory --------------------------------------------------------
 // int_ref_kernel's windows (the next 64 bits evaluated at once, the k-th uphill one drawing
@@ -170,7 +202,7 @@ static size_t ref_rows_lds(const DevGraph& g, int waves, bool lds_rows) {
 // and 12.3 or 14.5 ms at one wave; at 4,096 replicas of the larger graph int_ref_kernel's one
 // round of 16 waves beats two of 13).
 int int_ref_rows_waves(const DevGraph& g, int R, int cus, bool* lds_rows) {
-    if (!g.orows) return 0;
+    if (g.w0 == 0) return 0;
     const int per_cu = (R + cus - 1) / cus;
     auto cost = [&](int capacity, double base, double slope) {
         const int rounds = (per_cu + capacity - 1) / capacity;
@@ -433,7 +465,7 @@ static size_t sweep_rows_lds(const DevGraph& g, int waves, bool lds_rows) {
 // and 65 at 8,192).
 IntShape int_shape(const DevGraph& g, int R, int cus) {
     IntShape best{kIntSweep, 0};
-    if (!g.prows) return best;
+    if (g.w0 == 0) return best;
     const int per_cu = (R + cus - 1) / cus;
     auto cost = [&](int capacity, double base, double slope) {
         const int rounds = (per_cu + capacity - 1) / capacity;
