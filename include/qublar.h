@@ -147,6 +147,11 @@ typedef struct {
     double fp32_residual_err; /* max |r_carried - r_scratch_fp64| over rays and branches (FP32 carry) */
 } qb_report;
 
+/* The kernel that an anneal of n_branches with these options (NULL: the defaults) would run,
+   a static text: "ray_team", or one workgroup per branch, "ray_solo/bytes" and
+   "ray_solo/bits" by how its spins lie in LDS. For logs and tests; results do not depend on it. */
+int qb_anneal_kernel(qb_problem* p, int n_branches, const qb_anneal_opts* opts, const char** name);
+
 /* n_branches branches with seeds b + 1 + seed_offset annealed from all-zero x:
    branch_fractions (src/ising_recon.hpp:148-166) and anneal_branch (:121-144).
    Outputs (each nullable): branches n_branches x n_vars bytes (0/1), p_void n_vars
@@ -302,6 +307,12 @@ int qb_run_batch(qb_graph* g, const qb_schedule* b, uint64_t seed_base, int R, d
    in LDS up to 160 KB and in global memory beyond; the trajectory is the same either way. */
 int qb_run_batch_reference(qb_graph* g, const qb_schedule* b, uint64_t seed_base, int R, double updates_per_launch,
                            int8_t* s_out, int64_t* energy_out, qb_batch_report* rep);
+
+/* The kernel that qb_run_batch of R replicas would run (reference != 0: qb_run_batch_reference),
+   a static text: "int_sweep" (32-bit rows), or on 16-bit rows in LDS or L2 "int_wide/lds",
+   "int_wide/l2", "int_rows/lds", "int_rows/l2"; "int_ref", "int_ref_rows/lds", "int_ref_rows/l2".
+   For logs and tests; results do not depend on it. */
+int qb_run_batch_kernel(qb_graph* g, int R, int reference, const char** name);
 
 /* device_energies (ising_gpu.cuh:461-475): -cut of K states (K x n bytes, 0/1). */
 int qb_device_energies(qb_graph* g, const uint8_t* X, int K, int64_t* energy_out);

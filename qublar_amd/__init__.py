@@ -175,6 +175,7 @@ def lib():
             "qb_colour_problem": (i32, [C.POINTER(ProblemDesc), vp, vp, C.POINTER(i32)]),
             "qb_anneal_branches": (i32, [vp, C.POINTER(Schedule), i32, u64, C.POINTER(AnnealOpts), vp, vp, vp, vp,
                                          vp, C.POINTER(Report)]),
+            "qb_anneal_kernel": (i32, [vp, i32, C.POINTER(AnnealOpts), C.POINTER(C.c_char_p)]),
             "qb_energy": (i32, [vp, vp, i32, vp, vp, vp]),
             "qb_energy_noalloc": (i32, [vp, vp, i32, vp, vp, vp]),
             "qb_stage_create": (i32, [vp, C.POINTER(Schedule), i32, C.POINTER(AnnealOpts), C.POINTER(vp)]),
@@ -195,6 +196,7 @@ def lib():
             "qb_graph_colouring": (i32, [vp, vp, vp]),
             "qb_colour_graph": (i32, [C.POINTER(GraphDesc), vp, vp, C.POINTER(i32)]),
             "qb_run_batch": (i32, [vp, C.POINTER(Schedule), u64, i32, dbl, vp, vp, C.POINTER(BatchReport)]),
+            "qb_run_batch_kernel": (i32, [vp, i32, i32, C.POINTER(C.c_char_p)]),
             "qb_device_energies": (i32, [vp, vp, i32, vp]),
             "qb_run_batch_reference": (i32, [vp, C.POINTER(Schedule), u64, i32, dbl, vp, vp, C.POINTER(BatchReport)]),
             "qb_muon_scene_defaults": (i32, [C.POINTER(MuonScene)]),
@@ -420,6 +422,13 @@ class Problem:
         return dict(branches=br, p_void=pv, tri=tri, certainty=cert, energy=en,
                     report={f: getattr(rep, f) for f, _ in Report._fields_})
 
+    def anneal_kernel(self, n_branches, precision=FP64, workgroups=0, group_width=0):
+        """The kernel anneal_branches would run: "ray_team", "ray_solo/bytes" or "ray_solo/bits"."""
+        opts = AnnealOpts(precision, 0, workgroups, 0, group_width)
+        name = C.c_char_p()
+        _check(lib().qb_anneal_kernel(self.h, n_branches, C.byref(opts), C.byref(name)))
+        return name.value.decode()
+
     def freeze(self, margin):
         """freeze_provable_rock's frozen set on the device: (frozen uint8[n], rounds)."""
         fr = np.zeros(self.arrays.n_vars, np.uint8)
@@ -559,6 +568,12 @@ class Graph:
         out = {f: getattr(p, f) for f, _ in Plan._fields_}
         out["refused"] = p.refused.decode()
         return out
+
+    def run_batch_kernel(self, R, reference=False):
+        """The kernel run_batch (run_batch_reference) would run, with where its rows lie."""
+        name = C.c_char_p()
+        _check(lib().qb_run_batch_kernel(self.h, R, int(reference), C.byref(name)))
+        return name.value.decode()
 
     def run_batch(self, sched, seed_base, R, updates_per_launch=1e9):
         n_pad = self.plan()["n_pad"]

@@ -1081,27 +1081,51 @@ static int solo_for(qb_problem* P, const DevSolo** out) {
     return QB_OK;
 }
 
+// The checked options and launch shape of an anneal of R branches.
+struct AnnealShape {
+    qb_anneal_opts o{};
+    int group_width = 0, team_size = 0;   // of the team kernel
+    bool solo = false;                    // one workgroup per branch instead
+};
+
+static int anneal_shape(qb_problem* P, int R, const qb_anneal_opts* opts, AnnealShape& sh) {
+    if (R <= 0) return fail(QB_E_ARG, "n_branches must be positive (got %d)", R);
+    if (opts) sh.o = *opts;
+    const qb_anneal_opts& o = sh.o;
+    if (o.precision != QB_FP64 && o.precision != QB_FP32) return fail(QB_E_ARG, "precision must be QB_FP64 or QB_FP32");
+    if (o.recompute_every < 0 || o.sweeps_per_launch < 0 || o.workgroups < 0)
+        return fail(QB_E_ARG, "negative option");
+    if (o.group_width != 0 && o.group_width != 2 && o.group_width != 4 && o.group_width != 8 && o.group_width != 16)
+        return fail(QB_E_ARG, "group_width must be 0, 2, 4, 8 or 16 (got %d)", o.group_width);
+    sh.group_width = group_width_for(P, R, o.group_width, o.precision);
+    sh.team_size = team_size_for(o.workgroups, o.precision, sh.group_width, 0);
+    if (sh.team_size <= 0) return -sh.team_size;
+    sh.solo = solo_fits(P, o, R, 8 * sh.team_size);
+    return QB_OK;
+}
+
+extern "C" int qb_anneal_kernel(qb_problem* P, int n_branches, const qb_anneal_opts* opts, const char** name) {
+    if (!P || !name) return fail(QB_E_ARG, "qb_anneal_kernel: null argument");
+    AnnealShape sh;
+    if (int rc = anneal_shape(P, n_branches, opts, sh)) return rc;
+    *name = !sh.solo ? "ray_team"
+            : solo_spins_in_bits(P->n, P->n_rays, solo_wide_chains(P), sh.o.precision) ? "ray_solo/bits" : "ray_solo/bytes";
+    return QB_OK;
+}
+
 extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, uint64_t seed_offset,
                                   const qb_anneal_opts* opts, uint8_t* branches, float* p_void, uint8_t* tri,
                                   float* certainty, double* energy, qb_report* rep) {
     if (!P) return fail(QB_E_ARG, "qb_anneal_branches: null problem");
     int rc = check_schedule(s);
     if (rc) return rc;
-    if (R <= 0) return fail(QB_E_ARG, "n_branches must be positive (got %d)", R);
-    qb_anneal_opts o{};
-    if (opts) o = *opts;
-    if (o.precision != QB_FP64 && o.precision != QB_FP32) return fail(QB_E_ARG, "precision must be QB_FP64 or QB_FP32");
-    if (o.recompute_every < 0 || o.sweeps_per_launch < 0 || o.workgroups < 0)
-        return fail(QB_E_ARG, "negative option");
-    if (o.group_width != 0 && o.group_width != 2 && o.group_width != 4 && o.group_width != 8 && o.group_width != 16)
-        return fail(QB_E_ARG, "group_width must be 0, 2, 4, 8 or 16 (got %d)", o.group_width);
+    AnnealShape sh;
+    if ((rc = anneal_shape(P, R, opts, sh))) return rc;
+    const qb_anneal_opts& o = sh.o;
     const int total = s->anneal_sweeps + s->hold_sweeps;
-    const int n = P->n, nr = P->n_rays;
-    const int team_bw = group_width_for(P, R, o.group_width, o.precision);
-    const int team_size = team_size_for(o.workgroups, o.precision, team_bw, 0);
-    if (team_size <= 0) return -team_size;
-    const bool solo = solo_fits(P, o, R, 8 * team_size);
-    const int bw = solo ? 1 : team_bw;
+    const int n = P->n, nr = P->n_rays, team_size = sh.team_size;
+    const bool solo = sh.solo;
+    const int bw = solo ? 1 : sh.group_width;
     const int n_groups = (R + bw - 1) / bw;
     const size_t tsz = o.precision == QB_FP32 ? sizeof(float) : sizeof(double);
     const DevBatches* bt = nullptr;
@@ -1979,6 +2003,11 @@ static int bit_rows(qb_graph* G) {
     return QB_OK;
 }
 
+// force_global keeps the state in global memory, which int_sweep_kernel alone works on.
+static IntShape batch_shape(const qb_graph* G, int R) {
+    return G->lds_state ? int_shape(G->dev, R, G->cus) : IntShape{kIntSweep, 0};
+}
+
 extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_base, int R, double updates_per_launch,
                             int8_t* s_out, int64_t* energy_out, qb_batch_report* rep) {
     if (!G) return fail(QB_E_ARG, "qb_run_batch: null graph");
@@ -1992,8 +2021,7 @@ extern "C" int qb_run_batch(qb_graph* G, const qb_schedule* b, uint64_t seed_bas
     if ((rc = G->w_s.reserve(cells)) || (rc = G->w_f.reserve(cells * 4)) || (rc = G->w_e.reserve(sizeof(long long) * size_t(R))) ||
         (rc = G->w_sout.reserve(cells)) || (rc = G->w_beta.reserve(sizeof(double) * size_t(total))))
         return rc;
-    // force_global keeps the state in global memory
-    const IntShape sh = G->lds_state ? int_shape(G->dev, R, G->cus) : IntShape{kIntSweep, 0};
+    const IntShape sh = batch_shape(G, R);
     if (sh.kind != kIntSweep && (rc = position_rows(G))) return rc;
     const std::vector<double> beta = betas_of(*b);
     hipStream_t st = G->stream;
@@ -2088,6 +2116,25 @@ extern "C" int qb_run_batch_reference(qb_graph* G, const qb_schedule* b, uint64_
         rep->kernel_ms = ms;
         rep->launches = launches;
         rep->sweeps_per_launch = chunk;
+    }
+    return QB_OK;
+}
+
+extern "C" int qb_run_batch_kernel(qb_graph* G, int R, int reference, const char** name) {
+    if (!G || !name) return fail(QB_E_ARG, "qb_run_batch_kernel: null argument");
+    if (R <= 0) return fail(QB_E_ARG, "R must be positive (got %d)", R);
+    if (reference) {
+        bool lds_rows = false;
+        const int waves = int_ref_rows_waves(G->dev, R, G->cus, &lds_rows);
+        *name = waves == 0 ? "int_ref" : lds_rows ? "int_ref_rows/lds" : "int_ref_rows/l2";
+        return QB_OK;
+    }
+    switch (batch_shape(G, R).kind) {
+        case kIntWide: *name = "int_wide/lds"; break;
+        case kIntWideL2: *name = "int_wide/l2"; break;
+        case kIntRows: *name = "int_rows/lds"; break;
+        case kIntRowsL2: *name = "int_rows/l2"; break;
+        default: *name = "int_sweep"; break;
     }
     return QB_OK;
 }

@@ -272,6 +272,8 @@ struct DevSolo {
 };
 size_t solo_dynamic_lds(int n, int n_rays, int wide_chains, int precision, bool bits);
 size_t solo_lds_limit();
+// Whether a branch's spins lie in LDS as bits: as bytes they do not fit beside the residuals.
+bool solo_spins_in_bits(int n, int n_rays, int wide_chains, int precision);
 hipError_t launch_solo_blocks(const DevProblem& p, const SoloTile* tiles, const SlotDesc* desc, int n_tiles, void* blk,
                               SoloWide* wide, int n_wide, hipStream_t st);
 // Branches 0 .. R - 1, one workgroup each: x (R x n, u16, bit 0) and r (R x n_rays) receive

@@ -607,10 +607,14 @@ size_t solo_lds_limit() {
     return size_t(160) * 1024 - 2 * kSoloDraws * sizeof(Draw) - size_t(kSoloStepWaves) * kSoloPart * sizeof(double) - 64;
 }
 
+bool solo_spins_in_bits(int n, int n_rays, int wide_chains, int precision) {
+    return solo_dynamic_lds(n, n_rays, wide_chains, precision, false) > solo_lds_limit();
+}
+
 hipError_t launch_ray_solo(const DevProblem& p, const DevSolo& d, int precision, void* x, void* r, int R,
                            uint64_t seed_offset, const double* beta, int sb, int se, int recompute_every,
                            hipStream_t st) {
-    const bool bits = solo_dynamic_lds(p.n, p.n_rays, d.wide_chains, precision, false) > solo_lds_limit();
+    const bool bits = solo_spins_in_bits(p.n, p.n_rays, d.wide_chains, precision);
     const size_t lds = solo_dynamic_lds(p.n, p.n_rays, d.wide_chains, precision, bits);
     if (lds > solo_lds_limit()) return hipErrorInvalidValue;
     auto go = [&](auto zero, auto packed) -> hipError_t {
