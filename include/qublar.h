@@ -181,6 +181,9 @@ int qb_anneal_branches_reference(qb_problem* p, const qb_schedule* s, int n_bran
 int qb_anneal_branches_reference_split(qb_problem* p, const qb_schedule* s, int n_branches, uint64_t seed_offset,
                                        int sweeps_per_launch, uint8_t* branches, float* p_void, uint8_t* tri,
                                        float* certainty, double* energy, qb_report* rep);
+/* The kernel that anneals n_branches on the reference's own trajectory, a static text: "ray_ref", or
+   "ray_ref_lane" for many branches of short columns. For logs and tests; results do not depend on it. */
+int qb_anneal_reference_kernel(qb_problem* p, int n_branches, const char** name);
 
 /* The frozen set of freeze_provable_rock (src/ising_recon.hpp:187-205) on the device:
    frozen[i] = 1 (original bit order) where bit i is provably rock at `margin` nats. The

@@ -190,6 +190,7 @@ def lib():
                                                    C.POINTER(Report)]),
             "qb_anneal_branches_reference_split": (i32, [vp, C.POINTER(Schedule), i32, u64, i32, vp, vp, vp, vp, vp,
                                                          C.POINTER(Report)]),
+            "qb_anneal_reference_kernel": (i32, [vp, i32, C.POINTER(C.c_char_p)]),
             "qb_graph_create": (i32, [C.POINTER(GraphDesc), i32, C.POINTER(vp)]),
             "qb_graph_destroy": (i32, [vp]),
             "qb_graph_get_plan": (i32, [vp, C.POINTER(Plan)]),
@@ -427,6 +428,12 @@ class Problem:
         opts = AnnealOpts(precision, 0, workgroups, 0, group_width)
         name = C.c_char_p()
         _check(lib().qb_anneal_kernel(self.h, n_branches, C.byref(opts), C.byref(name)))
+        return name.value.decode()
+
+    def anneal_reference_kernel(self, n_branches):
+        """The kernel anneal_branches_reference would run: "ray_ref" or "ray_ref_lane"."""
+        name = C.c_char_p()
+        _check(lib().qb_anneal_reference_kernel(self.h, n_branches, C.byref(name)))
         return name.value.decode()
 
     def freeze(self, margin):

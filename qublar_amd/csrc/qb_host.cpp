@@ -332,6 +332,7 @@ struct qb_problem {
     DevBuf w_x, w_r, w_beta, w_bar, w_err, w_part, w_pv, w_tri, w_cert, w_br, w_data, w_prior, w_rerr, w_X, w_x16, w_rref,
         w_ref, w_rng, w_energy;
     int64_t ref_widest = 0;    // the most entries that one window of 64 bits has in dev.ref
+    double ref_lane = -1.0;    // ref_lane_from, < 0 until asked for
     int device = 0;   // the device current at creation: its stream, buffers and scratch
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     ~qb_problem() {
@@ -1478,6 +1479,44 @@ extern "C" int qb_stage_sweeps(const qb_stage* S, int* sweeps) {
 // leaves the split to the library (about a second at a few branches of the muon QUBO).
 constexpr double kRefFloatUpdatesPerLaunch = 33554432.0;
 
+// The branches per CU from which the reference's float trajectory runs on ray_ref_lane_kernel,
+// infinity where ray_ref_kernel is always the shorter. The lane kernel's time goes with its longest
+// columns and holds up to 28 waves a CU; the other's with its windows' instructions, eight
+// waves a CU, and least with ray-free bits, which it decides 64 at a time, and neighbours, which it
+// holds in registers. Measured at 64 to 3,000 bits, T = 20 and 1, uniform columns of k entries, ray_ref_kernel
+// over lane kernel, 4 neighbours: k = 1: 1.0 at 4 branches a CU, 1.5 at 8, 1.75 at 16; k = 3: 0.9, 1.4, 1.35;
+// k = 5: 0.8, 1.2, 1.0; k = 6: 0.7, 1.1, 0.95; k = 8: 0.6, 1.0, 0.8; k = 2 without neighbours 1.3 at 5 and 2.0
+// at 16, with ten 0.8 and 1.1; half of the bits ray-free 0.65 and 1.1; lengths of 1 to 8 as uniform 6.
+static double ref_lane_from(qb_problem* P) {
+    if (P->ref_lane >= 0.0) return P->ref_lane;
+    int64_t bits = 0;   // with entries
+    for (int p = 0; p < P->n; ++p) bits += P->col_ptr[size_t(p) + 1] > P->col_ptr[size_t(p)];
+    P->ref_lane = std::numeric_limits<double>::infinity();
+    if (bits > 0) {
+        const double k = 0.5 * (double(P->nnz) / double(bits) + P->max_entries);
+        const double neighbours = double(P->n_nbr) / P->n;
+        if (k <= 7.5 - 0.5 * neighbours) P->ref_lane = (3.1 + 0.5 * k + 0.35 * neighbours) * P->n / double(bits);
+    }
+    return P->ref_lane;
+}
+
+// Whether n_branches branches run on ray_ref_lane_kernel.
+static int ref_by_lane(qb_problem* P, int n_branches, bool& lane) {
+    int cus = 0;
+    if (int rc = device_cus(cus)) return rc;
+    lane = double(n_branches) > ref_lane_from(P) * cus;
+    return QB_OK;
+}
+
+extern "C" int qb_anneal_reference_kernel(qb_problem* P, int n_branches, const char** name) {
+    if (!P || !name) return fail(QB_E_ARG, "qb_anneal_reference_kernel: null argument");
+    if (n_branches <= 0) return fail(QB_E_ARG, "n_branches must be positive (got %d)", n_branches);
+    bool lane = false;
+    if (int rc = ref_by_lane(P, n_branches, lane)) return rc;
+    *name = lane ? "ray_ref_lane" : "ray_ref";
+    return QB_OK;
+}
+
 // The problem laid out in bit order (dev.ref), on the first anneal that reads it.
 static int ref_layout_for(qb_problem* P) {
     if (P->dev.ref.w) return QB_OK;
@@ -1542,7 +1581,9 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
                                     double(std::max(total, 1))));
     const int n_groups = (R + kGroup - 1) / kGroup;
     const int n_part = ray_energy_blocks(P->dev);
-    if ((rc = ref_layout_for(P)) || (rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
+    bool lane = false;
+    if ((rc = ref_by_lane(P, R, lane))) return rc;
+    if ((!lane && (rc = ref_layout_for(P))) || (rc = P->w_X.reserve(size_t(R) * size_t(std::max(n, 1)))) ||
         (rc = P->w_rref.reserve(sizeof(double) * size_t(R) * size_t(std::max(nr, 1)))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
         (rc = P->w_x.reserve(sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
@@ -1565,9 +1606,15 @@ extern "C" int qb_anneal_branches_reference_split(qb_problem* P, const qb_schedu
     QB_HIP(hipMemcpyAsync(P->w_beta.p, temp.data(), sizeof(double) * temp.size(), hipMemcpyHostToDevice, st));
     QB_HIP(hipEventRecord(P->ev0, st));
     int launches = 0;
-    for (int s0 = 0; s0 < total || launches == 0; s0 += per_launch, ++launches)
-        QB_HIP(launch_ray_ref(P->dev, P->ref_widest, R, seed_offset, P->w_beta.as<double>(), s0,
-                              std::min(total, s0 + per_launch), P->w_X.as<uint8_t>(), P->w_rref.as<double>(), P->w_rng.as<uint64_t>(), st));
+    for (int s0 = 0; s0 < total || launches == 0; s0 += per_launch, ++launches) {
+        const int s1 = std::min(total, s0 + per_launch);
+        if (lane)
+            QB_HIP(launch_ray_ref_lane(P->dev, R, seed_offset, P->w_beta.as<double>(), s0, s1, P->w_X.as<uint8_t>(),
+                                       P->w_rref.as<double>(), P->w_rng.as<uint64_t>(), st));
+        else
+            QB_HIP(launch_ray_ref(P->dev, P->ref_widest, R, seed_offset, P->w_beta.as<double>(), s0, s1,
+                                  P->w_X.as<uint8_t>(), P->w_rref.as<double>(), P->w_rng.as<uint64_t>(), st));
+    }
     QB_HIP(hipEventRecord(P->ev1, st));
     // the branches in the group masks of the read-out and energy kernels
     if (n > 0) QB_HIP(launch_pack_states(P->w_X.as<uint8_t>(), R, n, P->dev.pos_bit, P->w_x.as<uint16_t>(), st));

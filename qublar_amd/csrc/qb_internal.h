@@ -380,6 +380,9 @@ hipError_t launch_freeze_round(const DevProblem& p, const double* lb, double mar
 hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t entries, hipStream_t st);
 hipError_t launch_ray_ref(const DevProblem& p, int64_t widest, int R, uint64_t seed_offset, const double* temp,
                           int sweep_begin, int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
+// The same on the position-order rows, a lane a column: many branches of short columns.
+hipError_t launch_ray_ref_lane(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
+                               int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
 // The reference's own integer trajectory (wising::anneal), one wave per replica with its
 // state in LDS (n_pad * 5 bytes; four replicas per workgroup while that fits), or in global
 // memory when one replica's state exceeds kRefLdsLimit: temp[sweep] is the temperature,

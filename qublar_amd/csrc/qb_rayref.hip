@@ -1,5 +1,6 @@
-// qb_rayref.hip -- gfx950 kernel of the reference's own float trajectory (anneal_branch,
-// src/ising_recon.hpp:119-143).
+// qb_rayref.hip -- gfx950 kernels of the reference's own float trajectory (anneal_branch,
+// src/ising_recon.hpp:119-143): ray_ref_kernel, and ray_ref_lane_kernel for many branches of short
+// columns.
 //
 // Branch b anneals from x = 0, r = -d with seed b + 1 + seed_offset: bits in index order,
 // dE = local_field_dE (lin delta, then w (r a + a^2 / 2) per entry with a = a_k delta in CSR
@@ -345,6 +346,141 @@ __global__ void __launch_bounds__(64) ray_ref_kernel(DevProblem p, uint64_t seed
     if (lane == 0) sm[b] = st;
 }
 
+// Many branches of short columns: a lane walks its own bit's column, eight entries' loads in flight,
+// and the first accepted bit of a window is the loop's next flip. A flip of a bit with rays ends
+// the window; after a ray-free bit's flip the later lanes only sum their neighbour terms again
+// and decide anew. Spins are bytes in global memory. ray_ref_kernel's registers hold a CU to eight of
+// its waves; this one's leave room for 28, whose round trips to memory overlap, and a column of a few
+// entries is one such trip: 4,096 branches of 200 bits with three entries each, 20 sweeps at T = 20, take
+// 24.4 ms here and 32.3 there (16 branches 10.7 and 6.4). Where the line lies: ref_lane_from.
+__global__ void __launch_bounds__(256) ray_ref_lane_kernel(DevProblem p, int R, uint64_t seed_offset, const double* temp,
+                                                           int sweep_begin, int sweep_end, uint8_t* xs, double* rs,
+                                                           uint64_t* sm) {
+    const int w = int(threadIdx.x) / 64, lane = int(threadIdx.x) % 64;
+    const int b = int(blockIdx.x) * 4 + w;
+    if (b >= R) return;   // the whole wave leaves; waves never sync with each other
+    const int n = p.n;
+    uint8_t* x = xs + size_t(b) * size_t(n);
+    double* r = rs + size_t(b) * size_t(p.n_rays);
+    uint64_t st;
+    if (sweep_begin == 0) {
+        for (int i = lane; i < n; i += 64) x[i] = 0;
+        for (int k = lane; k < p.n_rays; k += 64) r[k] = -p.d[k];
+        st = (uint64_t(b) + 1u + seed_offset) * 0x2545F4914F6CDD1Dull + 1;
+    } else {
+        st = sm[b];
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t below = (uint64_t(1) << lane) - 1u;
+    for (int sweep = sweep_begin; sweep < sweep_end; ++sweep) {
+        const double T = temp[sweep];
+        const double nrT = T < 1e300 ? -1.0 / T : __builtin_nan("");   // NaN: every exponential exact
+        int i0 = 0;
+        while (i0 < n) {
+            const int i = i0 + lane;
+            const bool valid = i < n;
+            const int pos = valid ? p.bit_pos[i] : 0;
+            double dE = 0.0, base = 0.0;   // base: the sum up to the neighbour terms
+            const int xi = valid ? int(x[i]) : 0;
+            // each lane's column bounds and update order, kept for the flip
+            const int c0 = valid ? p.col_ptr[pos] : 0, c1 = valid ? p.col_ptr[pos + 1] : 0;
+            const int seq = valid ? int(p.seq_update[pos]) : 0;
+            constexpr int kChunk = 8;
+            if (valid) {
+                // eight entries' loads, then their residuals, in flight together; the sum
+                // itself stays in CSR order
+                const double delta = xi ? -1.0 : 1.0;
+                dE = p.lin[pos] * delta;
+                const int k1 = c1;
+                for (int kb = c0; kb < k1; kb += kChunk) {
+                    RayEnt e[kChunk];
+                    double rv[kChunk];
+#pragma unroll
+                    for (int u = 0; u < kChunk; ++u) e[u] = p.ent[min(kb + u, k1 - 1)];
+#pragma unroll
+                    for (int u = 0; u < kChunk; ++u) rv[u] = r[e[u].ray];
+#pragma unroll
+                    for (int u = 0; u < kChunk; ++u) {
+                        if (kb + u >= k1) break;
+                        const double a = double(e[u].a) * delta;
+                        dE += e[u].w * (rv[u] * a + 0.5 * a * a);
+                    }
+                }
+                base = dE;
+                const int q1 = p.nb_ptr[pos + 1];
+                for (int qb = p.nb_ptr[pos]; qb < q1; qb += kChunk) {
+                    int xv[kChunk];
+#pragma unroll
+                    for (int u = 0; u < kChunk; ++u) xv[u] = x[p.nb_bit[min(qb + u, q1 - 1)]];
+#pragma unroll
+                    for (int u = 0; u < kChunk; ++u) {
+                        if (qb + u >= q1) break;
+                        dE += p.lambda * (xv[u] != xi ? -1.0 : 1.0);
+                    }
+                }
+            }
+            // decisions of the lanes in todo (lanes >= lo) on the current state, the k-th
+            // uphill one drawing st + k gamma
+            uint64_t todo = ~uint64_t(0), m_up = 0, m_acc = 0;
+            auto decide = [&]() {
+                const bool mine = valid && ((todo >> lane) & 1u);
+                const bool up = mine && dE > 0.0;
+                m_up = __ballot(up) & todo;
+                bool acc = mine && dE <= 0.0;
+                if (up) acc = ref_accept(mix64(st + uint64_t(__popcll(m_up & below) + 1) * kGamma) >> 11, dE, T, nrT);
+                m_acc = __ballot(acc) & todo;
+            };
+            decide();
+            for (;;) {
+                if (m_acc == 0) {
+                    st += uint64_t(__popcll(m_up)) * kGamma;
+                    i0 += 64;
+                    break;
+                }
+                const int js = __builtin_ctzll(m_acc);
+                const uint64_t upto = js == 63 ? ~uint64_t(0) : (uint64_t(2) << js) - 1u;
+                st += uint64_t(__popcll(m_up & upto)) * kGamma;
+                const int fi = i0 + js;
+                const int k0 = __shfl(c0, js), k1 = __shfl(c1, js), seq_f = __shfl(seq, js);
+                const int xf = __shfl(xi, js);
+                const double delta = xf ? -1.0 : 1.0;
+                if (!seq_f) {
+                    for (int k = k0 + lane; k < k1; k += 64) r[p.ent[k].ray] += double(p.ent[k].a) * delta;
+                } else if (lane == 0) {   // a ray repeats in the column: its additions in CSR order
+                    for (int k = k0; k < k1; ++k) r[p.ent[k].ray] += double(p.ent[k].a) * delta;
+                }
+                if (lane == 0) x[fi] = uint8_t(xf ^ 1);
+                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+                __builtin_amdgcn_wave_barrier();
+                todo = ~upto;
+                if (k1 > k0 || todo == 0) {   // residuals changed (or the window is done)
+                    i0 = fi + 1;
+                    break;
+                }
+                // A ray-free bit flipped: no residual changed, so a later lane's sum up to its
+                // neighbour terms stands; only those terms are summed again, in order.
+                if (valid && ((todo >> lane) & 1u)) {
+                    dE = base;
+                    const int q1 = p.nb_ptr[pos + 1];
+                    for (int qb = p.nb_ptr[pos]; qb < q1; qb += kChunk) {
+                        int xv[kChunk];
+#pragma unroll
+                        for (int u = 0; u < kChunk; ++u) xv[u] = x[p.nb_bit[min(qb + u, q1 - 1)]];
+#pragma unroll
+                        for (int u = 0; u < kChunk; ++u) {
+                            if (qb + u >= q1) break;
+                            dE += p.lambda * (xv[u] != xi ? -1.0 : 1.0);
+                        }
+                    }
+                }
+                decide();
+            }
+        }
+    }
+    if (lane == 0) sm[b] = st;
+}
+
 // Zero entries: the layout's gaps and padding.
 __global__ void __launch_bounds__(256) ref_zero_kernel(RefLayout to, size_t entries) {
     for (size_t k = size_t(blockIdx.x) * 256 + threadIdx.x; k < entries; k += size_t(gridDim.x) * 256) {
@@ -386,11 +522,18 @@ hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t en
     return hipGetLastError();
 }
 
+hipError_t launch_ray_ref_lane(const DevProblem& p, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
+                               int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st) {
+    ray_ref_lane_kernel<<<unsigned((R + 3) / 4), 256, 0, st>>>(p, R, seed_offset, temp, sweep_begin, sweep_end, xs, rs,
+                                                               sm);
+    return hipGetLastError();
+}
+
 hipError_t launch_ray_ref(const DevProblem& p, int64_t widest, int R, uint64_t seed_offset, const double* temp, int sweep_begin,
                           int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st) {
     // a pass holds the widest window where it can: with fewer terms in LDS more branches share a
     // CU (4,096 branches of 100 bits and 500 entries, 20 sweeps at T = 20: 22.6 ms with five batches, 22.1
-    // with one; there a CU holds eight waves and their instructions bound it)
+    // with one)
     const int pass = kBatch * int(std::clamp<int64_t>((widest + kBatch - 1) / kBatch, 1, kPassBatches));
     const size_t terms = sizeof(double) * size_t(pass + 2 * kTail);
     const size_t mask = sizeof(uint64_t) * ((size_t(p.n) + 63) / 64);
