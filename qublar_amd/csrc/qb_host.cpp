@@ -1142,7 +1142,8 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
     }
     const int n_part = ray_energy_blocks(P->dev);
     const int n16 = (R + kGroup - 1) / kGroup;   // groups of the energy kernels
-    if ((rc = P->w_x.reserve(sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
+    if ((rc = P->w_x.reserve(solo ? solo_spin_bytes(n) * size_t(R)
+                                  : sizeof(uint16_t) * size_t(n_groups) * size_t(std::max(n, 1)))) ||
         (rc = P->w_r.reserve(tsz * size_t(n_groups) * size_t(std::max(nr, 1)) * size_t(bw))) ||
         (rc = P->w_beta.reserve(sizeof(double) * size_t(total))) ||
         (rc = P->w_bar.reserve(sizeof(unsigned) * (kBarWords + kTicketWords))) ||
@@ -1180,18 +1181,17 @@ extern "C" int qb_anneal_branches(qb_problem* P, const qb_schedule* s, int R, ui
     }
     QB_HIP(hipEventRecord(P->ev1, st));
     const bool want_outputs = p_void || tri || certainty || branches;
-    if (want_outputs)
-        QB_HIP(launch_ray_outputs(P->dev, P->w_x.as<uint16_t>(), n_groups, bw, R, P->w_pv.as<float>(),
-                                  P->w_tri.as<uint8_t>(), P->w_cert.as<float>(),
-                                  branches ? P->w_br.as<uint8_t>() : nullptr, st));
     const bool want_energy = energy || rep;
+    const uint16_t* x16 = bw == kGroup ? P->w_x.as<uint16_t>() : P->w_x16.as<uint16_t>();
+    if (solo && (want_outputs || want_energy)) QB_HIP(launch_solo_masks(P->w_x.p, n, R, P->w_x16.as<uint16_t>(), st));
+    if (want_outputs)
+        QB_HIP(launch_ray_outputs(P->dev, solo ? x16 : P->w_x.as<uint16_t>(), solo ? n16 : n_groups, solo ? kGroup : bw, R,
+                                  P->w_pv.as<float>(), P->w_tri.as<uint8_t>(), P->w_cert.as<float>(),
+                                  branches ? P->w_br.as<uint8_t>() : nullptr, st));
     if (want_energy) {
         QB_HIP(hipMemsetAsync(P->w_rerr.p, 0, sizeof(float), st));
-        const uint16_t* x16 = P->w_x.as<uint16_t>();
-        if (bw != kGroup) {
+        if (!solo && bw != kGroup)
             QB_HIP(launch_regroup(P->w_x.as<uint16_t>(), n, n_groups, bw, P->w_x16.as<uint16_t>(), st));
-            x16 = P->w_x16.as<uint16_t>();
-        }
         QB_HIP(launch_ray_energy(P->dev, x16, R, P->w_r.p, bw, o.precision, P->w_part.as<double>(), n_part,
                                  P->w_data.as<double>(), P->w_prior.as<double>(), P->w_rerr.as<float>(), st));
     }

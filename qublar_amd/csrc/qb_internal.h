@@ -276,11 +276,14 @@ size_t solo_lds_limit();
 bool solo_spins_in_bits(int n, int n_rays, int wide_chains, int precision);
 hipError_t launch_solo_blocks(const DevProblem& p, const SoloTile* tiles, const SlotDesc* desc, int n_tiles, void* blk,
                               SoloWide* wide, int n_wide, hipStream_t st);
-// Branches 0 .. R - 1, one workgroup each: x (R x n, u16, bit 0) and r (R x n_rays) receive
-// the state after sweep_end, and hold it on entry when sweep_begin > 0.
+// Branches 0 .. R - 1, one workgroup each: x (solo_spin_bytes(n) each: a bit a position) and
+// r (R x n_rays) receive the state after sweep_end, and hold it on entry when sweep_begin > 0.
+inline size_t solo_spin_bytes(int n) { return sizeof(uint32_t) * ((size_t(n) + 31) / 32); }
 hipError_t launch_ray_solo(const DevProblem& p, const DevSolo& d, int precision, void* x, void* r, int R,
                            uint64_t seed_offset, const double* beta, int sweep_begin, int sweep_end,
                            int recompute_every, hipStream_t st);
+// Those spins into masks of kGroup branches, as the read-out and energy kernels take them.
+hipError_t launch_solo_masks(const void* x, int n, int R, uint16_t* x16, hipStream_t st);
 
 // ---- launchers (qb_kernels.hip) ----
 // Writes every packed batch's block (DevBatches::blk) from its slot descriptors.

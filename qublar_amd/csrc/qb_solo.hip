@@ -399,7 +399,7 @@ __device__ __forceinline__ void wide_step(const DevProblem& p, const SoloState<T
 }  // namespace
 
 template <typename T, bool BITS>
-__global__ void __launch_bounds__(kSoloBlock) ray_solo_kernel(DevProblem p, DevSolo d, uint16_t* xs, T* rs,
+__global__ void __launch_bounds__(kSoloBlock) ray_solo_kernel(DevProblem p, DevSolo d, uint32_t* xs, T* rs,
                                                               uint64_t seed_offset, const double* beta,
                                                               int sweep_begin, int sweep_end, int recompute_every) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -411,20 +411,19 @@ __global__ void __launch_bounds__(kSoloBlock) ray_solo_kernel(DevProblem p, DevS
     const Spins<BITS> x{reinterpret_cast<unsigned char*>(r + p.n_rays + 1)};
     const int tid = int(threadIdx.x), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int branch = int(blockIdx.x);
-    uint16_t* xg = xs + size_t(branch) * size_t(p.n);
+    const int words = (p.n + 31) / 32;   // a branch's spins in memory, a bit each
+    uint32_t* xg = xs + size_t(branch) * size_t(words);
     T* rg = rs + size_t(branch) * size_t(p.n_rays);
     // the branch's state into LDS: x = 0, r = -d, or what the last launch left
     for (int k = tid; k < p.n_rays; k += kSoloBlock) r[k] = sweep_begin == 0 ? T(-p.d[k]) : rg[k];
     if (tid == 0) r[p.n_rays] = T(0);
     if constexpr (BITS) {
-        for (int w = tid; w < (p.n + 31) / 32; w += kSoloBlock) {
-            uint32_t m = 0;
-            if (sweep_begin > 0)
-                for (int b = 0; b < 32 && 32 * w + b < p.n; ++b) m |= uint32_t(xg[32 * w + b] & 1u) << b;
-            reinterpret_cast<uint32_t*>(x.x)[w] = m;
-        }
+        for (int w = tid; w < words; w += kSoloBlock) reinterpret_cast<uint32_t*>(x.x)[w] = sweep_begin > 0 ? xg[w] : 0u;
     } else {
-        for (int i = tid; i < p.n; i += kSoloBlock) x.x[i] = sweep_begin > 0 ? static_cast<unsigned char>(xg[i] & 1u) : 0;
+        for (int i = tid; i < p.n; i += kSoloBlock) x.x[i] = 0;
+        if (sweep_begin > 0)
+            for (int i = tid; i < p.n; i += kSoloBlock)
+                x.x[i] = static_cast<unsigned char>((xg[i >> 5] >> (i & 31)) & 1u);
     }
     const uint64_t branch_key = seed_offset + uint64_t(branch) + 1u;
     const bool stepper = wave < kSoloStepWaves;
@@ -535,8 +534,36 @@ __global__ void __launch_bounds__(kSoloBlock) ray_solo_kernel(DevProblem p, DevS
         }
     }
     __syncthreads();
+    int words_out = (p.n + 31) / 32, branch_out = int(blockIdx.x);
+    asm("" : "+s"(words_out), "+s"(branch_out));   // nothing of this is kept through the sweeps
+    uint32_t* x_out = xs + size_t(branch_out) * size_t(words_out);
     for (int k = tid; k < p.n_rays; k += kSoloBlock) rg[k] = r[k];
-    for (int i = tid; i < p.n; i += kSoloBlock) xg[i] = uint16_t(x.at(i));
+    if constexpr (BITS) {
+        for (int w = tid; w < words_out; w += kSoloBlock) x_out[w] = reinterpret_cast<const uint32_t*>(x.x)[w];
+    } else {
+        for (int i0 = wave * 64; i0 < p.n; i0 += kSoloBlock) {   // 64 spins a wave
+            const int i = i0 + lane;
+            const uint64_t m = __ballot(i < p.n && x.x[min(i, p.n - 1)] != 0);
+            const int w = i0 / 32 + lane;
+            if (lane < 2 && w < words_out) x_out[w] = uint32_t(lane == 0 ? m : m >> 32);
+        }
+    }
+}
+
+// The spins of R branches as the solo kernel leaves them into masks of kGroup branches.
+__global__ void __launch_bounds__(256) solo_masks_kernel(const uint32_t* xs, int n, int R, uint16_t* x16) {
+    const int pos = int(blockIdx.x * blockDim.x + threadIdx.x);
+    if (pos >= n) return;
+    const size_t words = size_t(n + 31) / 32;
+    const int b0 = int(blockIdx.y) * kGroup;
+    unsigned m = 0;
+#pragma unroll
+    for (int q = 0; q < kGroup; ++q) {
+        const int b = min(b0 + q, R - 1);
+        const unsigned v = (xs[size_t(b) * words + size_t(pos >> 5)] >> (pos & 31)) & 1u;
+        m |= (b0 + q < R ? v : 0u) << q;
+    }
+    x16[size_t(blockIdx.y) * size_t(n) + size_t(pos)] = uint16_t(m);
 }
 
 // One workgroup per tile: writes its chains' heads (planes of one granule per chain; a fourth
@@ -611,6 +638,12 @@ bool solo_spins_in_bits(int n, int n_rays, int wide_chains, int precision) {
     return solo_dynamic_lds(n, n_rays, wide_chains, precision, false) > solo_lds_limit();
 }
 
+hipError_t launch_solo_masks(const void* x, int n, int R, uint16_t* x16, hipStream_t st) {
+    const dim3 grid{unsigned((n + 255) / 256), unsigned((R + kGroup - 1) / kGroup)};
+    if (n > 0) solo_masks_kernel<<<grid, 256, 0, st>>>(static_cast<const uint32_t*>(x), n, R, x16);
+    return hipGetLastError();
+}
+
 hipError_t launch_ray_solo(const DevProblem& p, const DevSolo& d, int precision, void* x, void* r, int R,
                            uint64_t seed_offset, const double* beta, int sb, int se, int recompute_every,
                            hipStream_t st) {
@@ -624,7 +657,7 @@ hipError_t launch_ray_solo(const DevProblem& p, const DevSolo& d, int precision,
                                                  hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
         if (e != hipSuccess) return e;
         ray_solo_kernel<T, BITS><<<unsigned(R), kSoloBlock, lds, st>>>(
-            p, d, static_cast<uint16_t*>(x), static_cast<T*>(r), seed_offset, beta, sb, se, recompute_every);
+            p, d, static_cast<uint32_t*>(x), static_cast<T*>(r), seed_offset, beta, sb, se, recompute_every);
         return hipGetLastError();
     };
     if (bits) return precision == 1 ? go(0.0f, std::true_type{}) : go(0.0, std::true_type{});
