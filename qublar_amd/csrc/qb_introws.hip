@@ -195,35 +195,42 @@ static size_t ref_rows_lds(const DevGraph& g, int waves, bool lds_rows) {
            (lds_rows ? 2 * size_t((g.m_dir + 7) & ~7) : 0) + size_t(waves) * g.n_pad;
 }
 
-// Replicas per workgroup of int_ref_rows_kernel, 0 where int_ref_kernel is the shorter. Each
-// candidate runs R in rounds of what its LDS holds per CU (at most 16 waves here, 32 there), a
-// round of w waves taking about 0.51 + 0.022 w with the rows in LDS, 0.57 + 0.02 w with them
-// in L2, and 1 + 0.04 w in int_ref_kernel (measured at n = 800 and 2,000, degree 48: 6.4, 8.4
-// and 12.3 or 14.5 ms at one wave; at 4,096 replicas of the larger graph int_ref_kernel's one
-// round of 16 waves beats two of 13).
+// Replicas per workgroup of int_ref_rows_kernel, 0 where int_ref_kernel is the shorter, by the
+// estimated time of R in rounds of what a CU holds at a time, in units of int_ref_kernel's one wave.
+// There 32 waves or what its LDS holds run at 1 + 0.04 w; here workgroups of 1 to 16 replicas, as
+// many side by side as the LDS holds (32 waves at most), at a base + 0.022 w, the base by the mean row:
+// up to 32 entries (four rows at a time) 0.36 with the rows in LDS and 0.40 with them in L2, up to 64 0.51
+// and 0.59, longer ones 0.60 and 0.72. Measured at n = 800 to 8,000 (degree 8: 0.30 of int_ref_kernel's
+// time at one wave, 30: 0.40 and 0.46, 48: 0.50 and 0.57, 100: 0.67, 375: 0.75). Where rounds decide: 2,000
+// vertices of degree 100 at 14 replicas a CU, two rounds of 7 against one of 14, 10.1 against 8.9 ms;
+// of degree 48 the two rounds are the shorter (9.7 and 10.1); 1,500 of degree 375 at 18, 9.7 against 8.0.
 int int_ref_rows_waves(const DevGraph& g, int R, int cus, bool* lds_rows) {
     if (g.w0 == 0) return 0;
     const int per_cu = (R + cus - 1) / cus;
-    auto cost = [&](int capacity, double base, double slope) {
-        const int rounds = (per_cu + capacity - 1) / capacity;
-        return rounds * (base + slope * ((per_cu + rounds - 1) / rounds));
-    };
+    auto up = [](int a, int b) { return (a + b - 1) / b; };
     const size_t state = size_t(g.n_pad) * 5;
     if (state > kRefLdsLimit) return 0;
     const int held = 4 * state <= kRefLdsLimit ? int(std::min<size_t>(8, kRefLdsLimit / (4 * state))) * 4
                                                : int(kRefLdsLimit / state);
-    double best = cost(held, 1.0, 0.04);
+    const int old_rounds = up(per_cu, held);
+    double best = old_rounds * (1.0 + 0.04 * up(per_cu, old_rounds));
     int waves = 0;
+    const int64_t entries = g.m_dir, n = g.n;
     for (const bool in_lds : {true, false}) {
-        int fit = std::min(16, per_cu);
-        while (fit > 0 && ref_rows_lds(g, fit, in_lds) > kRefLdsLimit) --fit;
-        if (fit == 0) continue;
-        const double c = in_lds ? cost(fit, 0.51, 0.022) : cost(fit, 0.57, 0.02);
-        if (c < best) {
-            best = c;
-            const int rounds = (per_cu + fit - 1) / fit;
-            waves = (per_cu + rounds - 1) / rounds;
-            *lds_rows = in_lds;
+        const double base = entries <= 32 * n   ? (in_lds ? 0.36 : 0.40)
+                            : entries <= 64 * n ? (in_lds ? 0.51 : 0.59)
+                                                : (in_lds ? 0.60 : 0.72);
+        for (int w = std::min(16, per_cu); w > 0; --w) {
+            const size_t lds = ref_rows_lds(g, w, in_lds);
+            if (lds > kRefLdsLimit) continue;
+            const int groups = up(up(R, w), cus);   // of the fullest CU
+            const int rounds = up(groups, std::max(1, std::min(32 / w, int(kRefLdsLimit / lds))));
+            const double c = rounds * (base + 0.022 * (up(groups, rounds) * w));
+            if (c < best) {
+                best = c;
+                waves = w;
+                *lds_rows = in_lds;
+            }
         }
     }
     return waves;
@@ -459,8 +466,9 @@ static size_t sweep_rows_lds(const DevGraph& g, int waves, bool lds_rows) {
 // sweep, in us, over the rounds that R takes at what the LDS holds per CU. At one replica a
 // sweep takes about 0.35 per class + 0.045 per bit in int_sweep_kernel, 0.33 per 64 bits of a
 // class + 0.017 per bit in int_sweep_rows_kernel (1.28 times that with the rows in L2), and
-// 0.4 per step + 0.0035 per bit in int_wide_kernel; more waves per CU lengthen it by 4 to
-// 5.5% each, a second int_wide_kernel workgroup by 30%. Measured at n = 100 to 8,000, degree 8
+// 0.4 per step + 0.0035 per bit in int_wide_kernel (1.1 times that with the rows in L2: 2,000 vertices
+// of degree 48 at 16 replicas a CU take 152 us a sweep there and 129 in int_sweep_kernel); more
+// waves per CU lengthen it by 4 to 5.5% each, a second int_wide_kernel workgroup by 30%. Measured at n = 100 to 8,000, degree 8
 // to 48 (n = 800, degree 48: 37, 19.5 and 10.3 us at one replica, 42, 21 and 42 at 1,024, 97
 // and 65 at 8,192).
 IntShape int_shape(const DevGraph& g, int R, int cus) {
@@ -479,7 +487,7 @@ IntShape int_shape(const DevGraph& g, int R, int cus) {
         const size_t wide = wide_lds(g, in_lds) + kWideStatic;
         if (wide <= kRefLdsLimit) {
             const int capacity = 2 * wide <= kRefLdsLimit ? 2 : 1;
-            const double c = cost(capacity, 0.4 * g.n_steps + 0.0035 * g.n, 0.3);
+            const double c = (in_lds ? 1.0 : 1.1) * cost(capacity, 0.4 * g.n_steps + 0.0035 * g.n, 0.3);
             if (c < least) {
                 least = c;
                 best = IntShape{in_lds ? kIntWide : kIntWideL2, 0};

@@ -58,3 +58,18 @@ def test_integer_kernels():
     g = graph(90, 10)
     assert qa.Graph(qa.GraphArrays(g.n, g.eu, g.ev, np.arange(1, g.m + 1))).run_batch_kernel(5) == "int_sweep"
     assert qa.Graph(g, force_global=True).run_batch_kernel(5) == "int_sweep"
+
+
+@pytest.mark.parametrize("n,degree,R,kernel,reference", [
+    (2000, 100, 3584, None, "int_ref"),          # rows of 100 entries: two rounds of 7 waves against one of 14
+    (1500, 375, 4608, "int_sweep", "int_ref"),
+    (2000, 48, 4096, "int_sweep", "int_ref_rows/l2"),   # of 48 the two rounds are the shorter
+    (1000, 100, 4608, None, "int_ref_rows/l2"),  # two workgroups of nine side by side
+])
+def test_integer_rules_where_rounds_decide(n, degree, R, kernel, reference):
+    """On 256 CUs; each line is the measured shorter of the two."""
+    G = qa.Graph(qa.er_graph(n, degree / (n - 1), 5))
+    print(n, degree, R, flush=True)
+    assert G.run_batch_kernel(R, reference=True) == reference
+    if kernel:
+        assert G.run_batch_kernel(R) == kernel
