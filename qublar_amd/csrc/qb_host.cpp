@@ -2387,9 +2387,6 @@ extern "C" int qb_qubo_batch_create(const qb_qubo_batch_desc* d, qb_qubo_batch**
         hoff += n;
     }
     B->n_total = B->inst_pos.back();
-    hipDeviceProp_t prop;
-    if (int prc = device_props(prop)) return prc;
-    B->cus = prop.multiProcessorCount;
     // the rows sliced by 64 positions of each class, entry-major (padding: the bit itself, J = 0)
     std::vector<int32_t> ctile, tptr, tpos, tcol;
     std::vector<float> tJ;
@@ -2432,7 +2429,7 @@ extern "C" int qb_qubo_batch_create(const qb_qubo_batch_desc* d, qb_qubo_batch**
     }
     hipStream_t st = B->stream;
     int rc;
-    if ((rc = B->b_inst_pos.upload(B->inst_pos, st)) || (rc = B->b_inst_cls.upload(B->inst_cls, st)) ||
+    if ((rc = device_cus(B->cus)) || (rc = B->b_inst_pos.upload(B->inst_pos, st)) || (rc = B->b_inst_cls.upload(B->inst_cls, st)) ||
         (rc = B->b_cls.upload(B->cls_ptr, st)) || (rc = B->b_h.upload(hp, st)) || (rc = B->b_bit.upload(bit, st)) ||
         (rc = B->b_seed.upload(B->seed, st)) || (rc = B->b_ctile.upload(ctile, st)) ||
         (rc = B->b_tptr.upload(tptr, st)) || (rc = B->b_tpos.upload(tpos, st)) || (rc = B->b_tcol.upload(tcol, st)) || (rc = B->b_tJ.upload(tJ, st)))
