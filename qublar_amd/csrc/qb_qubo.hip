@@ -232,19 +232,20 @@ __global__ void __launch_bounds__(kQuboEnergyBlock) qubo_energy_kernel(DevQuboBa
         const bool valid = pos < q.tile_pos[t + 1];
         const uint32_t mi = valid ? mk[pos - bit0] >> r0 : 0u;
         double pair[kR] = {};
-        const int at = q.tile_ptr[t], end = q.tile_ptr[t + 1];
-        for (int i = at; i < end; i += 64 * kFlight) {
+        // unsigned: the last step of rows that end at the int32 limit runs past it
+        const unsigned at = unsigned(q.tile_ptr[t]), end = unsigned(q.tile_ptr[t + 1]);
+        for (unsigned i = at; i < end; i += 64 * kFlight) {
             int cj[kFlight];
             float wj[kFlight];
             uint32_t mj[kFlight];
 #pragma unroll
             for (int u = 0; u < kFlight; ++u) {
-                const int from = min(i + 64 * u, end - 64) + lane;
+                const unsigned from = min(i + 64u * u, end - 64u) + unsigned(lane);
                 cj[u] = q.tcol[from];
                 wj[u] = q.tJ[from];
             }
 #pragma unroll
-            for (int u = 0; u < kFlight; ++u) mj[u] = i + 64 * u < end ? mk[cj[u]] >> r0 : 0u;
+            for (int u = 0; u < kFlight; ++u) mj[u] = i + 64u * u < end ? mk[cj[u]] >> r0 : 0u;
 #pragma unroll
             for (int u = 0; u < kFlight; ++u)
 #pragma unroll
