@@ -36,8 +36,6 @@ struct BitEnt {
     float a;
 };
 
-// The float problem on the device, in colour-class position order: position p
-// holds original bit pos_bit[p]; class c is positions [cls_ptr[c], cls_ptr[c+1]).
 // The problem in bit order, as the reference's own trajectory walks it: a window is 64
 // consecutive bits. The entries lie column after column, a window's first at a multiple of
 // 256 (zeros fill the gaps), each with its bit modulo 64; in a block of 256 entries, k lies at
@@ -65,6 +63,8 @@ struct RefLayout {
 };
 constexpr int kRefNb = 8;
 
+// The float problem on the device, in colour-class position order: position p
+// holds original bit pos_bit[p]; class c is positions [cls_ptr[c], cls_ptr[c+1]).
 struct DevProblem {
     int n, n_rays, n_classes;
     int64_t nnz, n_nbr;
@@ -376,11 +376,12 @@ hipError_t launch_stage_outputs(const DevProblem& p, const uint16_t* x, int bw, 
 hipError_t launch_freeze_bound(const DevProblem& p, double* lb, hipStream_t st);
 hipError_t launch_freeze_round(const DevProblem& p, const double* lb, double margin, const uint8_t* frozen,
                                uint8_t* next, unsigned* changed, hipStream_t st);
+// Writes the layout of p (p.ref_start set) into `to`, `entries` long.
+hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t entries, hipStream_t st);
 // The reference's own float trajectory (anneal_branch): branch b's spins xs[b][bit order]
 // (bytes), residuals rs[b][ray] (FP64) and splitmix64 state sm[b] in global memory; one
 // launch runs sweeps [sweep_begin, sweep_end), the first starting from x = 0. `widest`: the most
 // entries of a window in RefLayout.
-hipError_t launch_ref_layout(const DevProblem& p, const RefLayout& to, size_t entries, hipStream_t st);
 hipError_t launch_ray_ref(const DevProblem& p, int64_t widest, int R, uint64_t seed_offset, const double* temp,
                           int sweep_begin, int sweep_end, uint8_t* xs, double* rs, uint64_t* sm, hipStream_t st);
 // The same on the position-order rows, a lane a column: many branches of short columns.

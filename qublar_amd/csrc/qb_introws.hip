@@ -6,7 +6,8 @@
 //                        src/ising_weighted.hpp:250-267), a wave per replica, several
 //                        replicas of a workgroup sharing the rows in LDS;
 //   int_wide_kernel      the colour-class trajectory (qb_run_batch), a workgroup per
-//                        replica, for few replicas.
+//                        replica, for few replicas;
+//   int_sweep_rows_kernel  the same with a wave per replica, for many.
 #include <algorithm>
 
 #include "qb_internal.h"
@@ -383,7 +384,8 @@ constexpr size_t kWideStatic = 2 * kWideDraws * sizeof(Draw) + (kWideBlock / 64)
 // A wave per replica, as in int_sweep_kernel, several of a workgroup sharing the 16-bit rows
 // in LDS, and an uphill move decided through the float exponential's band instead of the
 // FP64 exponential. Nothing is shared between waves after the rows are in. 8,192 replicas x
-// 1,000 sweeps at n = 800, degree 48: 93.7 -> 63.0 ms; the bound is vector issue (the draws).
+// 1,000 sweeps at n = 800, degree 48: 93.7 -> 63.0 ms; the bound is vector issue (an instruction
+// in 77% of the SIMDs' cycles; the LDS is active in 24%).
 template <bool LDS_ROWS>
 __global__ void __launch_bounds__(1024) int_sweep_rows_kernel(DevGraph g, int R, uint64_t seed_base, const double* beta,
                                                               int sweep_begin, int sweep_end, int init,

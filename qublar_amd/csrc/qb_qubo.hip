@@ -60,14 +60,17 @@ constexpr int word_shift() {
 // as acc + w does, and an unset neighbour -- or a padding entry, whose coupling is zero --
 // leaves acc (up to the sign of an exact zero, which no decision sees).
 //
-// The sums bound the sweep, instruction by instruction. With four replicas to a byte, a
+// The sums are most of a sweep's instructions. With four replicas to a byte, a
 // multiplication spreads the nibble to one bit a byte and each replica's x_j, as 0 or 2.0, is
 // one byte moved to the top of a double: two instructions per (entry, replica) where bit
 // field, conversion and FMA are three (the accumulators hold twice the sums). Rows padded to
 // their tile's longest need no test per entry, and a tile's steps are its own length (16, then
 // 8, 4, 2 and 1 entries), not whole steps of 16. 48 instances of 1,000 to 16,384 bits, degrees
 // 3 to 64, 8 to 32 replicas, 400 sweeps: 86.5 -> 53.7 ms. (x_j as any one exponent bit of a
-// double would save the moved byte too, but factors of 2^-511 and below slow the FMAs: 280.)
+// double would save the moved byte too, but factors of 2^-511 and below slow the FMAs: 280.) There,
+// with the long jobs halved, a CU with a job has a vector instruction in 47% of its SIMDs' cycles
+// and its LDS active in 18%, its waves waiting for the rows' and spins' loads in between; a CU
+// has a job 42% of the time.
 template <int RB, int N, int SHIFT, typename W>
 __device__ __forceinline__ void walk_row(const int* tcol, const float* tJ, const W* mk, double (&acc)[RB]) {
     const unsigned lane = threadIdx.x % 64;

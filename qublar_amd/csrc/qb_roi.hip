@@ -21,7 +21,7 @@
 // n fields at every state and took an exponential for each state needed about 70 and 100
 // vector instructions per state in the two passes; this needs about 4 and 10. A call with
 // n = 26 takes 0.13 ms (2.07 before), with n = 32 2.1 ms (33.6 before: 2.0e12 states/s), with
-// n = 36 28 ms.
+// n = 36 26 ms.
 //
 // The bound is vector issue. Results depend on n and the inputs alone.
 #include "qb_internal.h"

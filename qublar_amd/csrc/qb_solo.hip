@@ -29,7 +29,8 @@
 //
 // Measured, team kernel -> here (kernel and call): 1,964 bits x 960 rays, 8 branches, 250
 // sweeps, FP32 24.3 -> 5.4 ms (0.95 us a class); 24,633 bits x 8,640 rays, 16 branches, FP64
-// 64.7 -> 37.4 ms (3.0 us a class, bound by the vector instructions of one CU); at 256
+// 64.7 -> 37.4 ms (3.0 us a class; some instruction in 70% of its CUs' SIMD cycles, a vector
+// one in 47%, and the rest waits of two waves a SIMD at once); at 256
 // branches the same problems take 10.6 -> 1.0 and 15.6 -> 3.1 us a class.
 #include <type_traits>
 
